@@ -34,8 +34,7 @@ struct FwdArgs {
     int64_t qn, qh, qs, kn, kh, ks, on, oh, os;  // element strides of q/gate, k/v, out
     int N, H, Sq, Sk, D;
     float scale;
-    int bias_vec;  // bias rows are whole 16-byte vectors (Sk % 8 == 0), one head's bias < 2^31 bytes
-    int order;     // work-item order (ItemOrder)
+    int order;  // work-item order (ItemOrder)
     FastDiv fqt, fn, fh;  // division by the query tiles per (n, h), by N and by H (set at launch)
 };
 
@@ -48,6 +47,21 @@ struct FwdArgs {
 //   D = 32), which the pair reads together, and a run's bias is two heads';
 // - kOrderRows, for packed rows with H odd: the heads of one row together.
 enum ItemOrder { kOrderRows = 0, kOrderHeads = 1, kOrderHeadPairs = 2 };
+
+// How the bias tile of a wave reaches its lanes (set at launch by bias_mode):
+// - kBiasDma: through LDS by direct-to-LDS loads, where every bias row starts on a 4-byte boundary
+//   (Sk even): a 16-byte buffer load needs no more than dword alignment;
+// - kBiasDmaOdd: the same where Sk is odd, so that every second row starts 2 bytes past a dword
+//   boundary. The wave's two query blocks then take the rows of one parity each (block 0 the
+//   aligned ones), so that the 2-byte shift is known at compile time and costs no instruction;
+// - kBiasRegs: 2-byte loads of each lane's 16 keys, for what is left (a bias at an odd multiple of
+//   2 bytes with Sk even, or a head's bias of 2^31 bytes or more).
+// Every Sk % 8 != 0 used to run kBiasRegs, whose 32 2-byte loads a tile and lane set the kernel's
+// time: the gated packed forward at [139, 139, 4, 4, 16] took 33.4 us and takes 16.3 (by columns), a
+// triangle attention block of 381 residues (4 heads of 32, with its two projections) 354 and 152.
+// The mode is a template parameter, not a run-time branch: the kernel then holds one bias path
+// (133 VGPRs and no spills at D = 32 where it had 168 and 4).
+enum BiasMode { kBiasRegs = 0, kBiasDma = 1, kBiasDmaOdd = 2 };
 
 template <int DP>
 struct FwdTile {
@@ -78,33 +92,30 @@ __device__ __forceinline__ half8 zero8() {
 __device__ __forceinline__ half8 ld8(const half_t* p) { return *reinterpret_cast<const half8*>(p); }
 
 // 16 consecutive halfs from p, elements at or past `valid` as 0
-__device__ __forceinline__ H16 load_h16(const half_t* p, int valid, bool vec) {
+__device__ __forceinline__ H16 load_h16(const half_t* p, int valid) {
     H16 r;
-    if (vec && valid >= 16) {
-        r.lo = ld8(p);
-        r.hi = ld8(p + 8);
-    } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            r.lo[j] = j < valid ? p[j] : (half_t)0.f;
-            r.hi[j] = j + 8 < valid ? p[j + 8] : (half_t)0.f;
-        }
+    for (int j = 0; j < 8; ++j) {
+        r.lo[j] = j < valid ? p[j] : (half_t)0.f;
+        r.hi[j] = j + 8 < valid ? p[j + 8] : (half_t)0.f;
     }
     return r;
 }
 
-template <int DP, bool LSE, bool GATE, bool TRIM>
+template <int DP, bool LSE, bool GATE, bool TRIM, int BM>
 __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_fwd_kernel(FwdArgs a) {
     using T = FwdTile<DP>;
+    constexpr bool kVec = BM != kBiasRegs, kOdd = BM == kBiasDmaOdd;
     // two key tiles in flight: one being read by the MFMAs, the next being written
     // (at DP = 32 four unpadded arrays instead, one per tensor and buffer: below)
     __shared__ __attribute__((aligned(16))) half_t Ks2[DP == 32 ? 1 : 2][T::kBK * T::kKsLd];
     __shared__ __attribute__((aligned(16))) half_t Vs2[DP == 32 ? 1 : 2][T::kBK * T::kKsLd];
     constexpr int kD32 = DP == 32 ? T::kBK * 32 : 8;
     __shared__ __attribute__((aligned(16))) half_t K32a[kD32], K32b[kD32], V32a[kD32], V32b[kD32];
-    // where bias rows are whole 16-byte vectors: each wave's bias tiles (its 32 queries x 64 keys),
-    // two buffers, filled by direct-to-LDS loads (below)
-    __shared__ __attribute__((aligned(16))) half_t Bs[T::kWaves][2][4 * 520];
+    // each wave's bias tiles (its 32 queries x 64 keys), two buffers, filled by direct-to-LDS loads
+    // (below); with odd rows then the dword past the tile of each row of query block 1 (a load
+    // writes 64 of them)
+    __shared__ __attribute__((aligned(16))) half_t Bs[T::kWaves][2][4 * 520 + (kOdd ? 128 : 0)];
 
     const int item = xcd_item(blockIdx.x, gridDim.x);
     const int rest = fdiv(item, a.fqt), qt = item - rest * (int)a.fqt.d;
@@ -146,14 +157,21 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
         }
     }
 
-    // Q^T as the B operand of S^T: lane column q = q0w + 16 qb + r16, slots d = 32 ks + 8 g + j
+    // Q^T as the B operand of S^T: lane column q = query(qb), slots d = 32 ks + 8 g + j. The wave's
+    // queries are q0w + 16 qb + r16, or with odd bias rows, those of one parity per block: block 0
+    // takes the queries whose bias row starts on a dword boundary (q0w is even, so bias_par, the
+    // parity of the head's first element, decides which those are).
     const int q0w = q0 + wave * (T::kQB * 16);
+    const half_t* const bias_head = a.bias + (int64_t)h * a.Sq * a.Sk;
+    const int bias_par = kOdd ? __builtin_amdgcn_readfirstlane((int)((reinterpret_cast<uintptr_t>(bias_head) >> 1) & 1)) : 0;
+    const auto query_of = [&](int qb, int r) { return kOdd ? q0w + 2 * r + (qb ^ bias_par) : q0w + 16 * qb + r; };
+    const auto query = [&](int qb) { return query_of(qb, r16); };
     // (loaded after the first key tile's loads are issued, so that their latencies overlap)
     half8 qop[T::kQB][T::kKS];
     const auto load_q = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int qb = 0; qb < T::kQB; ++qb) {
-            const int gq = q0w + 16 * qb + r16;
+            const int gq = query(qb);
 #pragma unroll
             for (int ks = 0; ks < T::kKS; ++ks) {
                 const int d0 = 32 * ks + 8 * g;
@@ -239,14 +257,44 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
             while (keys) {
                 const uint32_t k = (uint32_t)__builtin_ctzll(keys);
                 keys &= keys - 1ull;
-                *reinterpret_cast<__attribute__((address_space(3))) half_t*>(row + ((2u * k) ^ kill_x)) = v;
+                uint32_t at = (2u * k) ^ kill_x;
+                if constexpr (kOdd) {
+                    // block 1's rows sit one element later; key 63's is in the dword past the tile
+                    if (lane >= 16) {
+                        at = (2u * k + 2u) ^ kill_x;
+                        if (k == 63) at = 4 * 1040 + 4 * (uint32_t)(lane & 15) - (1040 * (lane >> 3) + 128 * (lane & 7));
+                    }
+                }
+                *reinterpret_cast<__attribute__((address_space(3))) half_t*>(row + at) = v;
             }
         };
         put(~keep64 & inside, (half_t)kMaskedLogit);
         put(~keep64 & ~inside, (half_t)(-INFINITY));
     };
     constexpr int kKillMax = 8;  // most dead keys per tile that go through LDS stores
-    const auto stage = [&](auto vec, int buf, int k0, uint64_t keep) {
+    // With odd rows, tiles with more dead keys store them row by row instead (a lane per key, 32
+    // stores): block 1's bias registers are one element off the pairs that fix_bias works on.
+    const auto kill_rows_lds = [&](int bb, int k0, uint64_t keep64) {
+        if ((keep64 >> lane) & 1u) return;
+        const half_t v = k0 + lane < a.Sk ? (half_t)kMaskedLogit : (half_t)(-INFINITY);
+        lds_char* const base = (lds_char*)(&Bs[wv][bb][0]);
+        for (int R = 0; R < 32; ++R) {
+            const uint32_t x = 2u * (uint32_t)lane + (R >= 16 ? 2u : 0u);
+            const uint32_t at = x == 128u ? 4 * 1040 + 4 * (uint32_t)(R & 15)
+                                          : 1040 * (R >> 3) + 128 * (R & 7) + (x ^ (32u * (uint32_t)((R & 7) >> 1)));
+            *reinterpret_cast<__attribute__((address_space(3))) half_t*>(base + at) = v;
+        }
+    };
+    // the dead keys of a tile whose bias came through LDS, into it; the register path and, with
+    // aligned rows, tiles of more than kKillMax dead keys leave them to fix_bias
+    const auto kill_lds = [&](int bb, int k0, uint64_t keep64) {
+        if (__builtin_popcountll(~keep64) <= kKillMax) {
+            kill_bias_lds(bb, k0, keep64);
+        } else if constexpr (kOdd) {
+            kill_rows_lds(bb, k0, keep64);
+        }
+    };
+    const auto stage = [&](int buf, int k0, uint64_t keep) {
         if constexpr (DP == 32) {
             // the tile came by direct-to-LDS loads (below): once they have landed, each wave
             // zeroes the K rows of the masked keys in its own fragment block, and where its bias
@@ -256,9 +304,7 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
                 const int key = 16 * ((lane & 15) >> 2) + 4 * wv + (lane & 3);
                 if (!((keep >> key) & 1u))
                     *reinterpret_cast<half8*>((buf ? K32b : K32a) + 512 * wv + 8 * lane) = zero8();
-                if constexpr (decltype(vec)::value) {
-                    if (__builtin_popcountll(~keep) <= kKillMax) kill_bias_lds(buf, k0, keep);
-                }
+                if constexpr (kVec) kill_lds(buf, k0, keep);
             }
         } else {
             half_t* Ks = Ks2[buf];
@@ -290,10 +336,8 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
         const int range = __builtin_amdgcn_readfirstlane(rows * (int)a.ks * 2);
         const auto rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kb_base + kofs), 0, range, 0x00020000);
         const auto rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vb_base + kofs), 0, range, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rk, (__attribute__((address_space(3))) void*)((buf ? K32b : K32a) + 512 * wv), 16, kdma, 0, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rv, (__attribute__((address_space(3))) void*)((buf ? V32b : V32a) + 512 * wv), 16, vdma, 0, 0, 0);
+        dma_lds<16>(rk, (buf ? K32b : K32a) + 512 * wv, kdma);
+        dma_lds<16>(rv, (buf ? V32b : V32a) + 512 * wv, vdma);
         const auto rm = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(mrow + k0), 0, rows, 0x00020000);
         mbyte = __builtin_amdgcn_raw_buffer_load_b8(rm, (uint32_t)lane, 0, 0);
     };
@@ -308,7 +352,7 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
     // Gated at DP = 32: the last key tile loads, in place of a next tile, the wave's gate rows into
     // the idle buffer's regions of this wave (its K fragment block: query block 0, its V rows:
     // block 1), so the epilogue's gate reads are LDS reads whose memory latency the last tile
-    // covered. Slot l of block qb is query q0w + 16 qb + R (R = l / 4), 16-byte chunk
+    // covered. Slot l of block qb is query query_of(qb, R) (R = l / 4), 16-byte chunk
     // c = (l % 4) ^ (R / 4) % 4 of the row, at byte 16 l; rows past Sq and chunks past D read zeros.
     bool gate_lds = false;
     const auto dma_gate = [&](int buf) {
@@ -319,35 +363,33 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
                                                           0, range, 0x00020000);
 #pragma unroll
         for (int qb = 0; qb < T::kQB; ++qb) {
-            const uint32_t off = 8 * c < a.D ? (uint32_t)(((16 * qb + R) * a.qs + 8 * c) * 2) : 0x80000000u;
+            const uint32_t off = 8 * c < a.D ? (uint32_t)(((query_of(qb, R) - q0w) * a.qs + 8 * c) * 2) : 0x80000000u;
             half_t* dst = (qb == 0 ? (buf ? K32b : K32a) : (buf ? V32b : V32a)) + 512 * wv;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
+            dma_lds<16>(rg, dst, off);
         }
         // and the head's gate bias (D halfs) into the wave's idle bias buffer of that parity
         const auto rgb = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.gate_bias + (int64_t)h * a.D), 0,
                                                            a.D * 2, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rgb, (__attribute__((address_space(3))) void*)&Bs[wv][buf][0], 16,
-                                                 16u * (uint32_t)lane, 0, 0, 0);
+        dma_lds<16>(rgb, &Bs[wv][buf][0], 16u * (uint32_t)lane);
         gate_lds = true;
     };
     int gate_buf = 0;
 
     // bias of this lane's 16 keys k0 + 16 g .. +15 for its queries, in a register set per tile
-    // parity: loaded one key tile ahead where rows are not whole 16-byte vectors, else read from
-    // LDS at the start of the tile (below); when the tile comes up, a masked key's bias becomes
-    // the masked logit -1e4 and a key past Sk's -inf
+    // parity: loaded one key tile ahead on the register path, else read from LDS at the start of
+    // the tile (below); when the tile comes up, a masked key's bias becomes the masked logit -1e4
+    // and a key past Sk's -inf
     // (the register path's row pointers: brow, set where that path starts)
     const half_t* brow[T::kQB];
     const auto set_brow = [&]() {
 #pragma unroll
         for (int qb = 0; qb < T::kQB; ++qb) {
-            const int gq = q0w + 16 * qb + r16;
+            const int gq = query(qb);
             const int gqc = gq < a.Sq ? gq : a.Sq - 1;
-            brow[qb] = a.bias + (int64_t)h * a.Sq * a.Sk + (int64_t)gqc * a.Sk + 16 * g;
+            brow[qb] = bias_head + (int64_t)gqc * a.Sk + 16 * g;
         }
     };
-    // Where bias rows are whole 16-byte vectors (and a head's bias spans under 2^31 bytes) the
-    // bias goes through LDS: a lane's 16 keys of one query row are 32 bytes of a different row
+    // On the direct-to-LDS paths the bias goes through LDS: a lane's 16 keys of one query row are 32 bytes of a different row
     // for each of 16 lanes, so register loads of them touch 16 cache lines per instruction, which
     // measured a sixth of the kernel's time. Instead the wave loads its 32 x 64 bias tile with
     // four direct-to-LDS loads (buffer_load ... lds) from a buffer whose range is the head's bias
@@ -357,24 +399,43 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
     // 16-byte skew between loads put the 16 rows of each 16-lane read on distinct LDS banks. Rows past Sq lie past the buffer's range and read zeros (their
     // results are never stored); keys past Sk read the next row's values or zeros and become -inf
     // when their tile comes up.
-    const half_t* const bias_head = a.bias + (int64_t)h * a.Sq * a.Sk;
-    uint32_t bdma[4];
+    // With odd rows, row 8 m + r of the LDS tile is query query_of(m / 2, 8 (m % 2) + r), and a row
+    // of block 1 starts 2 bytes past a dword boundary: its loads start at that boundary, so key k
+    // is element k + 1 of the row and the last key of the tile lies in the dword past it, which a
+    // fifth load brings (lane i < 16: the dword of block 1's row i, at byte 4160 + 4 i). Buffer
+    // bounds are checked by dword; the range is rounded up to the dword that holds the head's last
+    // element.
+    uint32_t bdma[kOdd ? 5 : 4];
+    const char* const bias_base = reinterpret_cast<const char*>(bias_head) - 2 * bias_par;
+    const int bias_bytes = kOdd ? (a.Sq * a.Sk * 2 + 2 * bias_par + 3) & ~3 : a.Sq * a.Sk * 2;
     {
         const int r = lane >> 3, seg = (lane & 7) ^ (2 * (r >> 1));
-        bdma[0] = (uint32_t)(q0w + r) * (uint32_t)a.Sk * 2u + 16u * (uint32_t)seg;
+        if constexpr (kOdd) {
+            const uint32_t row2 = 2u * (uint32_t)a.Sk;  // bytes of a bias row
 #pragma unroll
-        for (int m = 1; m < 4; ++m) bdma[m] = bdma[0] + (uint32_t)m * 16u * (uint32_t)a.Sk;
+            for (int m = 0; m < 4; ++m)
+                bdma[m] = (uint32_t)query_of(m >> 1, 8 * (m & 1) + r) * row2 + 2u * (uint32_t)bias_par -
+                          2u * (uint32_t)(m >> 1) + 16u * (uint32_t)seg;
+            bdma[4] = lane < 16 ? (uint32_t)query_of(1, lane) * row2 + 2u * (uint32_t)bias_par - 2u + 128u : 0x80000000u;
+        } else {
+            bdma[0] = (uint32_t)(q0w + r) * (uint32_t)a.Sk * 2u + 16u * (uint32_t)seg;
+#pragma unroll
+            for (int m = 1; m < 4; ++m) bdma[m] = bdma[0] + (uint32_t)m * 16u * (uint32_t)a.Sk;
+        }
     }
     const auto dma_bias = [&](int k0, int bb) {
-        const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(bias_head + k0), 0,
-                                                          (a.Sq * a.Sk - k0) * 2, 0x00020000);
+        const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(bias_base + 2 * k0), 0,
+                                                          bias_bytes - 2 * k0, 0x00020000);
 #pragma unroll
         for (int m = 0; m < 4; ++m)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rb, (__attribute__((address_space(3))) void*)&Bs[wv][bb][520 * m], 16, bdma[m], 0, 0, 0);
+            dma_lds<16>(rb, &Bs[wv][bb][520 * m], bdma[m]);
+        if constexpr (kOdd)
+            dma_lds<4>(rb, &Bs[wv][bb][4 * 520], bdma[4]);
     };
-    // this lane's 16 keys of query row 16 qb + r16 from the wave's buffer bb: segments 2 g and
-    // 2 g + 1, adjacent in LDS
+    // this lane's 16 keys of its query in block qb from the wave's buffer bb: segments 2 g and
+    // 2 g + 1, adjacent in LDS; with odd rows the element after them too for block 1, whose 16 keys
+    // are elements 1 .. 16 of the 17
+    half_t bias_x = (half_t)0.f;
     const auto read_bias = [&](int bb, H16 (&b)[T::kQB]) {
 #pragma unroll
         for (int qb = 0; qb < T::kQB; ++qb) {
@@ -382,19 +443,19 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
             const half_t* p = &Bs[wv][bb][520 * m + 8 * (8 * r + ((2 * g) ^ (2 * (r >> 1))))];
             b[qb].lo = ld8(p);
             b[qb].hi = ld8(p + 8);
+            if constexpr (kOdd) {
+                if (qb == 1)
+                    bias_x = Bs[wv][bb][g == 3 ? 4 * 520 + 2 * r16 : 520 * m + 8 * (8 * r + ((2 * g + 2) ^ (2 * (r >> 1))))];
+            }
         }
     };
+    const auto bias_at = [&](const H16 (&b)[T::kQB], int qb, int kk) -> half_t {
+        const int e = kOdd ? kk + qb : kk;
+        return e < 8 ? b[qb].lo[e & 7] : e < 16 ? b[qb].hi[e & 7] : bias_x;
+    };
     const auto fetch_bias = [&](int k0, H16 (&b)[T::kQB]) {
-        if (a.bias_vec && k0 + T::kBK <= a.Sk) {
 #pragma unroll
-            for (int qb = 0; qb < T::kQB; ++qb) {
-                b[qb].lo = ld8(brow[qb] + k0);
-                b[qb].hi = ld8(brow[qb] + k0 + 8);
-            }
-        } else {
-#pragma unroll
-            for (int qb = 0; qb < T::kQB; ++qb) b[qb] = load_h16(brow[qb] + k0, a.Sk - (k0 + 16 * g), a.bias_vec);
-        }
+        for (int qb = 0; qb < T::kQB; ++qb) b[qb] = load_h16(brow[qb] + k0, a.Sk - (k0 + 16 * g));
     };
     const auto fix_bias = [&](int k0, H16 (&b)[T::kQB], uint64_t keep64) {
         if (k0 + T::kBK <= a.Sk) {
@@ -423,21 +484,21 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
     // covers only the loads it needs.
     uint64_t keep_cur = 0u;
     const int k_last = (k_end - 1) / T::kBK * T::kBK;
-    const auto tile = [&](auto vec, auto first, int k0, int buf, H16 (&bias16)[T::kQB],
+    const auto tile = [&](auto first, int k0, int buf, H16 (&bias16)[T::kQB],
                           H16 (&bias_next)[T::kQB]) __attribute__((always_inline)) {
         const half_t* Ks = DP == 32 ? (buf ? K32b : K32a) : Ks2[buf & (DP == 32 ? 0 : 1)];
         const half_t* Vs = DP == 32 ? (buf ? V32b : V32a) : Vs2[buf & (DP == 32 ? 0 : 1)];
         bool more = true;
         bool reg_fix = keep_cur != ~0ull;
         int k_next = k0 + T::kBK;
-        if constexpr (decltype(vec)::value) {
+        if constexpr (kVec) {
             // this tile's bias loads, issued a tile ago, are the only loads in flight: wait for
             // them (the compiler does not order LDS reads after direct-to-LDS loads by itself)
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             // (keys past Sk read as dead: their mask bytes load as zero)
-            reg_fix = keep_cur != ~0ull && __builtin_popcountll(~keep_cur) > kKillMax;
+            reg_fix = !kOdd && keep_cur != ~0ull && __builtin_popcountll(~keep_cur) > kKillMax;
             if constexpr (DP != 32) {
-                if (keep_cur != ~0ull && !reg_fix) kill_bias_lds(buf, k0, keep_cur);
+                if (keep_cur != ~0ull) kill_lds(buf, k0, keep_cur);
             }
             read_bias(buf, bias16);
             k_next = min(k0 + T::kBK, k_last);
@@ -486,8 +547,7 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int kk = 4 * kb + i;
-                        const half_t b = kk < 8 ? bias16[qb].lo[kk] : bias16[qb].hi[kk - 8];
-                        s[kb][qb][i] = fmaf(s[kb][qb][i], scale, (float)b);
+                        s[kb][qb][i] = fmaf(s[kb][qb][i], scale, (float)bias_at(bias16, qb, kk));
                     }
         };
         logits();
@@ -559,7 +619,7 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
 #pragma unroll
             for (int qb = 0; qb < T::kQB; ++qb) hot |= !(lt[qb] <= 64.f);
             if (__any(hot)) {
-                if constexpr (decltype(vec)::value) {
+                if constexpr (kVec) {
                     read_bias(buf, bias16);
                     if (reg_fix) fix_bias(k0, bias16, keep_cur);
                 }
@@ -586,7 +646,7 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
         // the other buffer was last read a tile ago, before the barrier that ended that tile
         if (more) {
             keep_cur = __ballot(mbyte != 0u);
-            stage(vec, buf ^ 1, k_next, keep_cur);
+            stage(buf ^ 1, k_next, keep_cur);
         }
         // at DP = 32 the next tile's K and V, loaded straight into LDS at the start of this tile,
         // have landed before the barrier after which every wave reads them (the compiler also
@@ -651,9 +711,9 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
     };
 
     H16 biasA[T::kQB], biasB[T::kQB];
-    const auto run = [&](auto vec) __attribute__((always_inline)) {
+    const auto run = [&]() __attribute__((always_inline)) {
         fetch_kv(0, 0);
-        if constexpr (decltype(vec)::value) {
+        if constexpr (kVec) {
             dma_bias(0, 0);
         } else {
             set_brow();
@@ -667,25 +727,19 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
                 return;
             }
         }
-        stage(vec, 0, 0, keep_cur);
+        stage(0, 0, keep_cur);
         __syncthreads();
-        tile(vec, std::true_type{}, 0, 0, biasA, biasB);
+        tile(std::true_type{}, 0, 0, biasA, biasB);
         for (int k0 = T::kBK; k0 < k_end; k0 += 2 * T::kBK) {
-            tile(vec, std::false_type{}, k0, 1, biasB, biasA);
-            if (k0 + T::kBK < k_end) tile(vec, std::false_type{}, k0 + T::kBK, 0, biasA, biasB);
+            tile(std::false_type{}, k0, 1, biasB, biasA);
+            if (k0 + T::kBK < k_end) tile(std::false_type{}, k0 + T::kBK, 0, biasA, biasB);
         }
         // the last tile's bias loads (of itself, unused) land before the workgroup's LDS is freed
-        if constexpr (decltype(vec)::value) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if constexpr (kVec) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     };
-    if (k_end > 0) {
-        if (a.bias_vec) {
-            run(std::true_type{});
-        } else {
-            run(std::false_type{});
-        }
-    }
+    if (k_end > 0) run();
 
-    // epilogue: lane g holds d = (DP/4) g .. +DP/4 of query q0w + 16 qb + r16. Gated, out =
+    // epilogue: lane g holds d = (DP/4) g .. +DP/4 of query query(qb). Gated, out =
     // acc / (l (1 + 2^(-(gate + gate_bias) log2 e))): one reciprocal per element covers both the
     // softmax normalisation and the sigmoid, and -gate_bias log2 e is formed once per lane.
     float ngb[DP / 32][8];
@@ -701,7 +755,7 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
     }
 #pragma unroll
     for (int qb = 0; qb < T::kQB; ++qb) {
-        const int gq = q0w + 16 * qb + r16;
+        const int gq = query(qb);
         const float l = wave_xor_sum4(l_run[qb]);
         if (gq >= a.Sq) continue;
         if constexpr (LSE) {
@@ -744,6 +798,15 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
     }
 }
 
+// BiasMode of a bias [H, Sq, Sk]. Direct-to-LDS loads take 32-bit offsets within a head's bias, and
+// the swizzled rows past Sq must not wrap: heads of 2^31 bytes or more go through registers.
+static int bias_mode(const void* bias, int64_t Sq, int64_t Sk) {
+    if (Sq * Sk * 2 >= ((int64_t)1 << 31) - 4) return kBiasRegs;
+    const uintptr_t at = reinterpret_cast<uintptr_t>(bias);
+    if (Sk % 2 == 0) return at % 4 == 0 ? kBiasDma : kBiasRegs;
+    return at % 2 == 0 ? kBiasDmaOdd : kBiasRegs;
+}
+
 template <int DP, bool LSE, bool GATE, bool TRIM>
 static int launch_fwd(hipStream_t stream, int device, const FwdArgs& a) {
     using T = FwdTile<DP>;
@@ -760,9 +823,13 @@ static int launch_fwd(hipStream_t stream, int device, const FwdArgs& a) {
     b.fqt = fast_div(qt);
     b.fn = fast_div(a.N);
     b.fh = fast_div(a.H);
+    const int bm = bias_mode(a.bias, a.Sq, a.Sk);
     stage_mark(stream, 0);
-    hipLaunchKernelGGL((attn_fwd_kernel<DP, LSE, GATE, TRIM>), dim3((unsigned)grid),
-                       dim3(T::kThreads), 0, stream, b);
+#define CLK_FWD(BM_)                                                                               \
+    if (bm == BM_) hipLaunchKernelGGL((attn_fwd_kernel<DP, LSE, GATE, TRIM, BM_>), dim3((unsigned)grid), \
+                                      dim3(T::kThreads), 0, stream, b);
+    CLK_FWD(kBiasRegs) CLK_FWD(kBiasDma) CLK_FWD(kBiasDmaOdd)
+#undef CLK_FWD
     stage_mark(stream, 1);
     return launch_status("attention");
 }
@@ -845,7 +912,6 @@ extern "C" int clk_attention_fwd(clk_stream stream, int32_t device, const clk_bu
     a.out = static_cast<half_t*>(out->data);
     a.lse = want_lse ? static_cast<float*>(lse->data) : nullptr;
     a.scale = scale;
-    a.bias_vec = Sk % 8 == 0 && aligned16(a.bias) && (int64_t)Sq * Sk * 2 < ((int64_t)1 << 31);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     return want_lse ? dispatch_fwd<true, false, false>(s, device, a)
                     : dispatch_fwd<false, false, false>(s, device, a);
@@ -899,7 +965,6 @@ static int packed_common(clk_stream stream, int32_t device, const clk_buffer* p,
     a.out = static_cast<half_t*>(out->data);
     a.lse = nullptr;
     a.scale = scale;
-    a.bias_vec = S % 8 == 0 && aligned16(a.bias) && (int64_t)S * S * 2 < ((int64_t)1 << 31);
     a.order = H % 2 == 0 ? kOrderHeadPairs : kOrderRows;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (lims) {

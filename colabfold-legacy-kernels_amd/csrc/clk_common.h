@@ -103,6 +103,19 @@ __device__ __forceinline__ half8 lds_operand_tr(At at, int g, int lane16, int co
     return half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
+// A direct-to-LDS buffer load of BYTES (16 or 4) per lane: lane l's bytes at offset `off` of the
+// buffer land at dst + BYTES l, dst uniform across the wave; offsets past the buffer's range write
+// zeros. Counted by vmcnt like any load. (The 16-byte form is a gfx950 builtin that hipcc's host
+// pass rejects, there without a message.)
+template <int BYTES, typename Rsrc>
+__device__ __forceinline__ void dma_lds(Rsrc rsrc, void* dst, uint32_t off) {
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)dst, BYTES, off, 0, 0, 0);
+#else
+    (void)rsrc, (void)dst, (void)off;
+#endif
+}
+
 // Pin v as an fp32 register value, so its later rounding to fp16 is a separate step that the
 // compiler cannot fold into the multiply producing v (v_fma_mixlo_f16 rounds once). Every
 // template variant of a kernel then rounds alike, as the reference rounds its fp32 dS.
