@@ -43,7 +43,7 @@ __device__ __forceinline__ half8 fzero8() {
 __device__ __forceinline__ half8 fld8(const half_t* p) { return *reinterpret_cast<const half8*>(p); }
 __device__ __forceinline__ void fst8(half_t* p, half8 v) { *reinterpret_cast<half8*>(p) = v; }
 // A streaming (nontemporal) 16-byte store, for outputs that no later kernel of the op reads back
-// soon; measured faster for the wide outputs of ln_projection at c = 128 and ln_gdp, slower for
+// soon; measured faster for the wide outputs of ln_projection at c = 128, slower for
 // ln_projection at c = 64, where two workgroups share a CU.
 __device__ __forceinline__ void fst8_nt(half_t* p, half8 v) {
     __builtin_nontemporal_store(v, reinterpret_cast<half8*>(p));
@@ -864,8 +864,8 @@ __global__ __launch_bounds__(TH) void ln_gdp_kernel(LnGdpArgs a) {
                 }
             const int rows_left = a.M - (m0 + 16 * g);
             if (vec && rows_left >= 16) {
-                fst8_nt(dst, lo);
-                fst8_nt(dst + 8, hi);
+                fst8(dst, lo);
+                fst8(dst + 8, hi);
             } else {
 #pragma unroll
                 for (int t = 0; t < 16; ++t)
@@ -875,7 +875,7 @@ __global__ __launch_bounds__(TH) void ln_gdp_kernel(LnGdpArgs a) {
     }
 }
 
-// The same op for M % 8 == 0 (16-byte channel-major stores), with a tile body that is straight-line
+// The same op with a tile body that is straight-line
 // code, so that no wait for a load also waits for the stores issued before it (vmcnt counts
 // loads and stores in issue order, and the compiler's count is only as good as its weakest path):
 // - the next tile's mask rows are fetched with its x rows, and the keep decision is taken from
@@ -888,7 +888,21 @@ __global__ __launch_bounds__(TH) void ln_gdp_kernel(LnGdpArgs a) {
 //   the hardware drops, so every tile issues the same stores and no branch skips them;
 // - each wave owns CBW column blocks, fixed at compile time, with their biases in registers.
 // Offsets are 32-bit: the launcher requires P/2 * M * 2 bytes < 2^31.
-template <int K, int PH, int TH, bool BF>
+//
+// With M % 8 == 0 (RAG false) every channel's row of M results starts on a 16-byte boundary. Other M
+// (RAG, as with any odd number of residues) leave it on a 4-byte boundary, which a buffer store of
+// several dwords needs no more than, or for odd M and odd channels 2 bytes past one. A lane of such
+// a channel then stores its rows 16 g + 1 .. 16 g + 16 (the last from the lane group after it):
+// the eight dwords are formed with one align instruction each, whose shift is 0 for the other
+// channels. Per column block the stores are 4, 3 and 1 dwords (the last dropped where it would
+// reach into the next tile) and 2 bytes for the rows left over at the tile's ends. The one tile
+// that M cuts short stores 2 bytes at a time, after the loop.
+// Plain stores, not nontemporal ones: a store instruction writes 16-byte pieces of 16 channels, which
+// L2 must gather into whole lines. With nontemporal stores M = 262144 takes the same time, but where
+// the channels' rows do not start on 128-byte lines they double the kernel's: 99.1 and 52.6 us at
+// M = 145160, 155 and 48.6 at M = 145161 (K = P/2 = 128; the latter 149 us before RAG, when such M
+// ran ln_gdp_kernel).
+template <int K, int PH, int TH, bool BF, bool RAG>
 __global__ __launch_bounds__(TH) void ln_gdp_fast_kernel(LnGdpArgs a) {
     constexpr int KS = K / 32, TW = TH / kWave, NB = PH / 8, CBW = NB / TW;
     static_assert(NB % TW == 0, "whole column blocks per wave");
@@ -927,10 +941,18 @@ __global__ __launch_bounds__(TH) void ln_gdp_fast_kernel(LnGdpArgs a) {
     // 8-row chunks are all in or all out since M % 8 == 0; those past M are replaced at use)
     RowTile<K, kTileRows, TH> xt;
     half8 mlo, mhi;
+    // (RAG: rows past M read zeros, but for the one that shares row M - 1's dword)
+    const auto rmask = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.mask), 0,
+                                                         ((uint32_t)a.M * 2u + 3u) & ~3u, 0x00020000);
     const auto fetch = [&](int t) {
         const int r0 = t * kTileRows + 16 * g;
-        mlo = fld8(a.mask + min(r0, a.M - 8));
-        mhi = fld8(a.mask + min(r0 + 8, a.M - 8));
+        if constexpr (RAG) {
+            mlo = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rmask, (uint32_t)r0 * 2u, 0, 0));
+            mhi = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rmask, (uint32_t)r0 * 2u + 16u, 0, 0));
+        } else {
+            mlo = fld8(a.mask + min(r0, a.M - 8));
+            mhi = fld8(a.mask + min(r0 + 8, a.M - 8));
+        }
         constexpr int TPR = RowTile<K, kTileRows, TH>::kTPR;
         const int row = threadIdx.x / TPR, part = threadIdx.x % TPR;
         const int m = min(t * kTileRows + row, a.M - 1);
@@ -945,7 +967,14 @@ __global__ __launch_bounds__(TH) void ln_gdp_fast_kernel(LnGdpArgs a) {
     half8 mvlo, mvhi;
     const auto decide = [&](int t) {
         const int r0 = t * kTileRows + 16 * g;
-        const half8 klo = r0 < a.M ? mlo : fzero8(), khi = r0 + 8 < a.M ? mhi : fzero8();
+        half8 klo = r0 < a.M ? mlo : fzero8(), khi = r0 + 8 < a.M ? mhi : fzero8();
+        if constexpr (RAG) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                klo[e] = r0 + e < a.M ? klo[e] : (half_t)0.f;
+                khi[e] = r0 + 8 + e < a.M ? khi[e] : (half_t)0.f;
+            }
+        }
         mvlo = __builtin_elementwise_max(klo, fzero8());
         mvhi = __builtin_elementwise_max(khi, fzero8());
         const bool live = __builtin_reduce_max(__builtin_elementwise_max(mvlo, mvhi)) > (half_t)0.f;
@@ -955,7 +984,8 @@ __global__ __launch_bounds__(TH) void ln_gdp_fast_kernel(LnGdpArgs a) {
         const bool any_live = __any(live), any_zero = __any(zero);
         return any_live ? (int)kCompute : any_zero ? (int)kPadding : (int)kSkip;
     };
-    const auto gemm_store = [&](int t, int work) {
+    const auto gemm_store = [&](int t, int work, auto cut) {
+        constexpr bool kCut = decltype(cut)::value;  // (RAG) the tile that M cuts short
         const int m0 = t * kTileRows;
         half8 xop[4][KS];
 #pragma unroll
@@ -963,7 +993,7 @@ __global__ __launch_bounds__(TH) void ln_gdp_fast_kernel(LnGdpArgs a) {
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) xop[rb][ks] = fld8(Xf + frag(rb, ks, KS, lane));
         const bool zero_out = work == kPadding;
-        const int rows_left = a.M - (m0 + 16 * g);  // <= 0, 8 or >= 16
+        const int rows_left = a.M - (m0 + 16 * g);  // without RAG <= 0, 8 or >= 16
         const bool st_lo = work != kSkip && rows_left >= 8, st_hi = work != kSkip && rows_left >= 16;
 #pragma unroll
         for (int j = 0; j < CBW; ++j) {
@@ -1004,9 +1034,34 @@ __global__ __launch_bounds__(TH) void ln_gdp_fast_kernel(LnGdpArgs a) {
             const bool is_left = 16 * cb < PH;
             const uint32_t off = ((uint32_t)(is_left ? col : col - PH) * (uint32_t)a.M + (uint32_t)(m0 + 16 * g)) * 2u;
             const auto rs = is_left ? rl : rr;
-            // aux 2: nontemporal
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, lo), rs, st_lo ? off : kDrop, 0, 2);
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, hi), rs, st_hi ? off + 16u : kDrop, 0, 2);
+            if constexpr (kCut) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    __builtin_amdgcn_raw_buffer_store_b16(
+                        __builtin_bit_cast(unsigned short, e < 8 ? lo[e & 7] : hi[e & 7]), rs,
+                        work != kSkip && e < rows_left ? off + 2u * e : kDrop, 0, 0);
+            } else if constexpr (RAG) {
+                using u32x3 = unsigned int __attribute__((ext_vector_type(3)));
+                const u32x4 dl = __builtin_bit_cast(u32x4, lo), dh = __builtin_bit_cast(u32x4, hi);
+                const uint32_t d[9] = {dl[0], dl[1], dl[2], dl[3], dh[0], dh[1], dh[2], dh[3],
+                                       (uint32_t)__shfl_down((int)dl[0], 16)};
+                const uint32_t odd = (uint32_t)col & (uint32_t)a.M & 1u;
+                uint32_t o[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = __builtin_amdgcn_alignbit(d[e + 1], d[e], 16u * odd);
+                const bool st = work != kSkip;
+                const uint32_t at = st ? off + 2u * odd : kDrop;
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4{o[0], o[1], o[2], o[3]}, rs, at, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b96(u32x3{o[4], o[5], o[6]}, rs, at + 16u, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(o[7], rs, odd && g == 3 ? kDrop : at + 28u, 0, 0);
+                // rows 0 and 63 of the tile, alone in their dwords
+                const bool end = odd && (g == 0 || g == 3) && st;
+                __builtin_amdgcn_raw_buffer_store_b16((unsigned short)(g == 0 ? d[0] : d[7] >> 16), rs,
+                                                      end ? off + (g == 0 ? 0u : 30u) : kDrop, 0, 0);
+            } else {
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, lo), rs, st_lo ? off : kDrop, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, hi), rs, st_hi ? off + 16u : kDrop, 0, 0);
+            }
         }
     };
 
@@ -1019,8 +1074,14 @@ __global__ __launch_bounds__(TH) void ln_gdp_fast_kernel(LnGdpArgs a) {
     __syncthreads();
     for (;;) {
         const int nt = t + G;
+        if constexpr (RAG) {
+            if ((t + 1) * kTileRows > a.M) {  // the last tile of all
+                gemm_store(t, work, std::true_type{});
+                break;
+            }
+        }
         fetch(min(nt, tiles - 1));
-        gemm_store(t, work);
+        gemm_store(t, work, std::false_type{});
         if (nt >= tiles) break;
         t = nt;
         work = decide(t);
@@ -1709,10 +1770,11 @@ static int ln_gdp_launch(const LnGdpArgs& a, int64_t M, int64_t K, int64_t P, hi
     const size_t lds = (size_t)(2 * P * K + kTileRows * K) * 2 + 2 * K * 4;
     const int64_t tiles = (M + kTileRows - 1) / kTileRows;
     const dim3 grid(persistent_grid(tiles, lds));
-    if (M % 8 == 0 && P / 2 * M * 2 < (int64_t{1} << 31)) {  // 16-byte channel-major stores, 32-bit offsets
+    if (P / 2 * M * 2 < (int64_t{1} << 31) - 64) {  // 32-bit offsets
 #define CLK_GDP_FAST(K_, PH_)                                                                          \
     if (K == K_ && P / 2 == PH_) {                                                                     \
-        const auto kern = ln_gdp_fast_kernel<K_, PH_, gdp_threads<K_>(), BF>;                          \
+        const auto kern = M % 8 == 0 ? ln_gdp_fast_kernel<K_, PH_, gdp_threads<K_>(), BF, false>       \
+                                     : ln_gdp_fast_kernel<K_, PH_, gdp_threads<K_>(), BF, true>;       \
         if (int st = launch_fused("ln_gdp", kern, grid, lds, s, &a, 0)) return st;                     \
         stage_mark(s, 0);                                                                              \
         hipLaunchKernelGGL(kern, grid, dim3(gdp_threads<K_>()), lds, s, a);                            \
