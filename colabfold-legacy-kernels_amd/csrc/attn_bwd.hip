@@ -54,7 +54,8 @@ struct BwdArgs {
     // loads is one contiguous 1 KB sweep
     half_t* bfrag;
     // workspace [2][windows][N][H][Sk][D]: with more than one query window, each window's fp32
-    // dK (unscaled) and dV sums over its queries, added up in window order by dkdv_sum_kernel
+    // dK (unscaled) and dV sums over its queries, added up in window order by dkdv_sum_kernel; the
+    // register kernel's windows, launched one after another, keep one running sum, [2][N][H][Sk][D]
     float* dkv;
     int N, H, Sq, Sk, D;
     int SqA, SkA;    // Sq rounded up to 32, Sk rounded up to 64
@@ -64,6 +65,9 @@ struct BwdArgs {
     int chunks;
     int wtiles;      // 32-query tiles per query window of the dK/dV kernel
     int windows;     // query windows: ceil(Sq / 32 / wtiles)
+    // this launch's window of the register dK/dV kernel: its first 32-query tile, and whether it is
+    // the first and the last one of the call
+    int wt0, wfirst, wlast;
     float scale;
     float c1;    // scale log2e, or 1 where |scale log2e| is below 1e-30
     float c1s;   // c1 / log2e: scale, or the stand-in's 1 / log2e
@@ -231,10 +235,8 @@ __global__ __launch_bounds__(DqTile<DP>::kThreads, DP == 32 ? 4 : 1) void attn_b
         const auto rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kb_base + kofs), 0, range, 0x00020000);
         const auto rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vb_base + kofs), 0, range, 0x00020000);
         const uint32_t koff = (keep >> dkey) & 1u ? kvdma : 0x80000000u;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rk, (__attribute__((address_space(3))) void*)((buf ? K32b : K32a) + 512 * wv), 16, koff, 0, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rv, (__attribute__((address_space(3))) void*)((buf ? V32b : V32a) + 512 * wv), 16, kvdma, 0, 0, 0);
+        dma_lds<16>(rk, (buf ? K32b : K32a) + 512 * wv, koff);
+        dma_lds<16>(rv, (buf ? V32b : V32a) + 512 * wv, kvdma);
     };
     const auto fetch_kv = [&](int k0, int buf, uint64_t keep) {
         if constexpr (DP == 32) {
@@ -857,7 +859,7 @@ __global__ __launch_bounds__(256 * QG) void attn_bwd_dkdv_kernel(BwdArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------
-// dK, dV and the dBias partials where D == 32 and Sq <= 32 QT (QT = 4 launches it; the same
+// dK, dV and the dBias partials where D <= 32 and Sq <= 32 QT (QT = 4 launches it; the same
 // layout in query parts, attn_bwd_dkdv_reg3_kernel, serves QT 8 and 12): the same
 // products and lane layout as attn_bwd_dkdv_kernel, arranged so that the dBias partial never
 // leaves registers. A workgroup of eight waves owns 64 keys of one head and a chunk of batch
@@ -914,7 +916,7 @@ template <int QT, bool DBIAS>
 __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
     using T = RegTile<QT>;
     static_assert(QT % 4 == 0 && QT <= 12, "whole steps of two tiles per half");
-    constexpr int DP = T::DP, HT = T::HT, kSteps = T::kSteps, kSub = T::kSub, kOs = T::kOs;
+    constexpr int HT = T::HT, kSteps = T::kSteps, kSub = T::kSub, kOs = T::kOs;
     constexpr int kBuf = T::kBuf, SqB = T::SqB, kBRow = T::kBRow;
     __shared__ __attribute__((aligned(16))) float bias_l[65 * kBRow];  // rows: 64 keys, masked
     __shared__ __attribute__((aligned(16))) half_t lds[2 * kBuf];
@@ -954,7 +956,8 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
     // rows crow and crow + 16 at a fixed column
     const int ti = wave >> 1, tensor = wave & 1, sqh = ti >> 1, si = ti & 1;
     const int crow = lane >> 2, ccol = (lane & 3) * 8;
-    const uint32_t cvoff = (uint32_t)((crow * DP + ccol) * 2);
+    const int D = a.D;
+    const uint32_t cvoff = ccol < D ? (uint32_t)((crow * D + ccol) * 2) : 0x80000000u;
     const int cdst0 = (2 * sqh + si) * kSub + tensor * kOs + 2 * reg_word(perm_row(crow, 8), ccol);
     const int cdst1 = (2 * sqh + si) * kSub + tensor * kOs + 2 * reg_word(perm_row(crow + 16, 8), ccol);
     const half_t* const csrc = tensor ? a.dout : a.q;
@@ -971,9 +974,9 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
         const int64_t nh = row_nh(pass);
         const int q0 = 32 * (sqh * HT + 2 * step + si);
         const auto rs = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<half_t*>(csrc + (nh * a.Sq + q0) * DP), 0, max(a.Sq - q0, 0) * DP * 2, 0x00020000);
+            const_cast<half_t*>(csrc + (nh * a.Sq + q0) * D), 0, max(a.Sq - q0, 0) * D * 2, 0x00020000);
         chk[0] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rs, cvoff, 0, 0));
-        chk[1] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rs, cvoff + 16u * DP * 2u, 0, 0));
+        chk[1] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rs, cvoff + 32u * (uint32_t)D, 0, 0));
         if (wave == 0) {
             const int tg = (qt_t >> 1) * HT + 2 * step + (qt_t & 1);
             const auto rq = __builtin_amdgcn_make_buffer_rsrc(
@@ -994,11 +997,11 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
     // offsets fixed for the kernel
     half8 kopn, vopn;
     uint32_t mbn = 0u;
-    const uint32_t kvoff = (uint32_t)((kin ? key : 0) * DP + 8 * g) * 2u, moff = (uint32_t)(kin ? key : 0);
+    const uint32_t kvoff = 8 * g < D ? (uint32_t)((kin ? key : 0) * D + 8 * g) * 2u : 0x80000000u, moff = (uint32_t)(kin ? key : 0);
     const auto fetch_kv = [&](int pass) {
         const int64_t nh = row_nh(pass);
-        const auto rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.k + nh * a.Sk * DP), 0, a.Sk * DP * 2, 0x00020000);
-        const auto rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.v + nh * a.Sk * DP), 0, a.Sk * DP * 2, 0x00020000);
+        const auto rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.k + nh * a.Sk * D), 0, a.Sk * D * 2, 0x00020000);
+        const auto rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.v + nh * a.Sk * D), 0, a.Sk * D * 2, 0x00020000);
         const auto rm = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.kmask + (int64_t)row_n(pass) * a.Sk), 0, a.Sk, 0x00020000);
         mbn = (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(rm, moff, 0, 0);
         kopn = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rk, kvoff, 0, 0));
@@ -1111,7 +1114,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
             __syncthreads();
         }
 
-        if (qh == 0 && kin) {
+        if (qh == 0 && kin && 8 * g < D) {
             // half 0 + half 1, then lane holds d = 8 g .. + 8 of its key (a masked key's dS,
             // and so dK, is 0)
             const float4* r = red + ((T::kSlots == 2 ? (pass & 1) : 0) * 4 + kg) * 4 * 64 + lane;
@@ -1120,7 +1123,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
                                  acck[1][0] + k1.x, acck[1][1] + k1.y, acck[1][2] + k1.z, acck[1][3] + k1.w};
             const float vs[8] = {accv[0][0] + v0.x, accv[0][1] + v0.y, accv[0][2] + v0.z, accv[0][3] + v0.w,
                                  accv[1][0] + v1.x, accv[1][1] + v1.y, accv[1][2] + v1.z, accv[1][3] + v1.w};
-            const int64_t off = (((int64_t)n * a.H + h) * a.Sk + key) * DP + 8 * g;
+            const int64_t off = (((int64_t)n * a.H + h) * a.Sk + key) * D + 8 * g;
             half8 ok, ov;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -1147,7 +1150,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------
-// The register dK/dV kernel in query parts, D = 32: for QT = 12 (256 < Sq <= 384) twelve waves
+// The register dK/dV kernel in query parts, D <= 32: for QT = 12 (256 < Sq <= 384) twelve waves
 // at three per SIMD, key group w % 4 by query third w / 4 (four tiles each, two per step), so the
 // dBias partial is 32 registers per lane and the kernel fits 168 VGPRs; for QT = 8 (128 < Sq <=
 // 256) sixteen waves at four per SIMD, key group w % 4 by query quarter w / 4 (two tiles each, one
@@ -1161,6 +1164,14 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
 // buffers (and the two term buffers) are separate arrays with compile-time selection, so the
 // compiler can tell that the step's LDS reads do not alias the loads in flight and does not wait
 // for them. Everything else is attn_bwd_dkdv_reg_kernel's.
+//
+// Sq > 384 runs it in query windows (WIN), one launch after another, each QT tiles from wt0 on: a
+// window's dK / dV sums of a row start from the fp32 running sum that the window before left in the
+// workspace (loaded during the row's last step, through a range of no bytes where there is none) and
+// go back there, or, in the last window, to dk and dv. The traffic of the running sum (16 N H Sk D
+// bytes a window after the first) runs beside the products. At [640, 4, 640, 32] windows of 12 and 8
+// tiles take 871 us (rocprofv3); the LDS-partial kernel in two windows of 10, with a pass that adds up
+// their sums, took 992 + 207.
 // ------------------------------------------------------------------------------------------
 template <int QT>
 struct PartTile {
@@ -1169,14 +1180,14 @@ struct PartTile {
     static constexpr int kTPS = QT == 12 ? 2 : 1;        // tiles per part and step
 };
 
-template <int QT, bool DBIAS>
+template <int QT, bool DBIAS, bool WIN>
 __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn_bwd_dkdv_reg3_kernel(BwdArgs a) {
     static_assert(QT == 12 || QT == 8, "query parts of two tiles per step (QT 12) or one (QT 8)");
     constexpr int kParts = PartTile<QT>::kParts, kTPS = PartTile<QT>::kTPS, kNT = PartTile<QT>::kThreads;
-    constexpr int DP = 32, TT = QT / kParts;  // tiles per part
+    constexpr int TT = QT / kParts;  // tiles per part
     constexpr int kSteps = TT / kTPS;
     static_assert(kSteps == 2, "buffer parity alternates by step within a row");
-    constexpr int kTile = 32 * DP, kOs = kTile + 64, kSub = kOs + kTile;
+    constexpr int kTile = 32 * 32, kOs = kTile + 64, kSub = kOs + kTile;
     constexpr int kBuf = kParts * kTPS * kSub;  // halfs of a step: [part][tile]
     constexpr int kQTerms = kParts * kTPS * 16; // float4 slots of a step's query terms
     constexpr int SqB = 32 * QT;
@@ -1204,6 +1215,9 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
     const int key = kblk * 64 + klocal;
     const bool kin = key < a.Sk;
     const float c1s = a.c1s;
+    const int D = a.D;
+    const int wt0 = WIN ? a.wt0 : 0;  // the window's first tile
+    const int SqR = WIN ? a.SqB : SqB;  // transposed-bias row length
 
     if (tid < 192) reinterpret_cast<float4*>(tid < 96 ? qterms0 + 512 : qterms1 + 128)[tid] = make_float4(0.f, 0.f, 0.f, 0.f);
 
@@ -1218,7 +1232,8 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
     for (int i = 0; i < 2; ++i) {
         const int R = 16 * i + (lane >> 2), p = lane & 3;
         const int x = 8 * ((R >> 2) & 3) + 4 * (R >> 4) + (R & 3);
-        dvoff[i] = (uint32_t)((x * DP + 8 * (p ^ ((R >> 2) & 3))) * 2);
+        const int col = 8 * (p ^ ((R >> 2) & 3));
+        dvoff[i] = col < D ? (uint32_t)((x * D + col) * 2) : 0x80000000u;
     }
     const int dst_off = (kTPS * sq3 + si) * kSub + tensor * kOs;
     const half_t* const csrc = tensor ? a.dout : a.q;
@@ -1235,22 +1250,19 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
     const auto dma_s = [&](int pass, int step, int buf) {
         const int64_t nh = row_nh(pass);
         if (stager) {
-            const int q0 = 32 * (sq3 * TT + kTPS * step + si);
+            const int q0 = 32 * (wt0 + sq3 * TT + kTPS * step + si);
             const auto rs = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<half_t*>(csrc + (nh * a.Sq + q0) * DP), 0, max(a.Sq - q0, 0) * DP * 2, 0x00020000);
+                const_cast<half_t*>(csrc + (nh * a.Sq + q0) * D), 0, max(a.Sq - q0, 0) * D * 2, 0x00020000);
             half_t* dst = (buf ? lds1 : lds0) + dst_off;
 #pragma unroll
             for (int i = 0; i < 2; ++i)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    rs, (__attribute__((address_space(3))) void*)(dst + 512 * i), 16, dvoff[i], 0, 0, 0);
+                dma_lds<16>(rs, dst + 512 * i, dvoff[i]);
         }
         if (wave * kWave < kQTerms) {
-            const int tg = (qt_t / kTPS) * TT + kTPS * step + (qt_t % kTPS);
+            const int tg = wt0 + (qt_t / kTPS) * TT + kTPS * step + (qt_t % kTPS);
             const auto rq = __builtin_amdgcn_make_buffer_rsrc(
                 const_cast<float*>(a.qstat + nh * a.SqA * 2), 0, a.SqA * 2 * 4, 0x00020000);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rq, (__attribute__((address_space(3))) void*)((buf ? qterms1 : qterms0) + 256 * wave), 16,
-                qL < kQTerms ? ((uint32_t)(64 * tg) + qt_f) * 4u : 0x80000000u, 0, 0, 0);
+            dma_lds<16>(rq, (buf ? qterms1 : qterms0) + 256 * wave, qL < kQTerms ? ((uint32_t)(64 * tg) + qt_f) * 4u : 0x80000000u);
         }
     };
 
@@ -1258,11 +1270,11 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
     // offsets fixed for the kernel
     half8 kopn, vopn;
     uint32_t mbn = 0u;
-    const uint32_t kvoff = (uint32_t)((kin ? key : 0) * DP + 8 * g) * 2u, moff = (uint32_t)(kin ? key : 0);
+    const uint32_t kvoff = 8 * g < D ? (uint32_t)((kin ? key : 0) * D + 8 * g) * 2u : 0x80000000u, moff = (uint32_t)(kin ? key : 0);
     const auto fetch_kv = [&](int pass) {
         const int64_t nh = row_nh(pass);
-        const auto rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.k + nh * a.Sk * DP), 0, a.Sk * DP * 2, 0x00020000);
-        const auto rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.v + nh * a.Sk * DP), 0, a.Sk * DP * 2, 0x00020000);
+        const auto rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.k + nh * a.Sk * D), 0, a.Sk * D * 2, 0x00020000);
+        const auto rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.v + nh * a.Sk * D), 0, a.Sk * D * 2, 0x00020000);
         const auto rm = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.kmask + (int64_t)row_n(pass) * a.Sk), 0, a.Sk, 0x00020000);
         mbn = (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(rm, moff, 0, 0);
         kopn = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rk, kvoff, 0, 0));
@@ -1285,14 +1297,14 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
     // the workgroup's bias, fp16: rows kblk 64 .. + 63 and the masked-logit row SkA
     {
         constexpr int kFill = (65 * (SqB / 4) + kNT - 1) / kNT;
-        const float* src = a.biast + (int64_t)h * (a.SkA + 1) * SqB;
+        const float* src = a.biast + (int64_t)h * (a.SkA + 1) * SqR + 32 * wt0;
 #pragma unroll
         for (int f = 0; f < kFill; ++f) {
             const int idx = tid + kNT * f;
             if (idx < 65 * (SqB / 4)) {
                 const int r = idx / (SqB / 4), c4 = idx - r * (SqB / 4);
                 const int srow = r < 64 ? kblk * 64 + r : a.SkA;
-                const float4 v = *reinterpret_cast<const float4*>(src + (int64_t)srow * SqB + 4 * c4);
+                const float4 v = *reinterpret_cast<const float4*>(src + (int64_t)srow * SqR + 4 * c4);
                 *reinterpret_cast<half4*>(bias_l + r * kBRow + 4 * c4) =
                     half4{(half_t)(v.x * (1.f / kLog2e)), (half_t)(v.y * (1.f / kLog2e)),
                           (half_t)(v.z * (1.f / kLog2e)), (half_t)(v.w * (1.f / kLog2e))};
@@ -1317,10 +1329,24 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
             acck[db] = float4v{0.f, 0.f, 0.f, 0.f};
         }
         fetch_kv(pass + 1);
+        float4 run[WIN ? 4 : 1];  // the running sums of the windows before: dK, dV of d = 8 g .. + 8
 
 #pragma unroll
         for (int st = 0; st < kSteps; ++st) {
             const int par = st & 1;  // kSteps is even
+            if constexpr (WIN) {
+                if (st == kSteps - 1) {
+                    const int64_t plane = (int64_t)a.N * a.H * a.Sk * D, nh = (int64_t)n * a.H + h;
+                    const int bytes = q3 == 0 && !a.wfirst ? a.Sk * D * 4 : 0;
+                    const uint32_t off = kin && 8 * g < D ? (uint32_t)(key * D + 8 * g) * 4u : 0x80000000u;
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        const auto rr = __builtin_amdgcn_make_buffer_rsrc(a.dkv + t * plane + nh * a.Sk * D, 0, bytes, 0x00020000);
+                        run[2 * t] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rr, off, 0, 0));
+                        run[2 * t + 1] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rr, off + 16u, 0, 0));
+                    }
+                }
+            }
             // the next step's tiles into the other buffer, whose last reads ended at the barrier
             dma_s(pass + (st + 1) / kSteps, (st + 1) % kSteps, par ^ 1);
             const half_t* buf = (par ? lds1 : lds0) + q3 * kTPS * kSub;
@@ -1385,27 +1411,6 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
                 soft(0);
                 dvdk(0);
             }
-#ifdef CLK_REG3_SGB
-            // tile 0's reads and products; tile 1's reads; tile 1's products each beside a quarter
-            // of tile 0's softmax; tile 0's transposed reads; its dV / dK products each beside a
-            // quarter of tile 1's softmax; tile 1's transposed reads and products
-            __builtin_amdgcn_sched_group_barrier(0x100, 9, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 9, 0);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-#endif
             if (st == kSteps - 1 && q3 > 0) {
                 float4* r = red + ((q3 - 1) * 4 + kg) * 4 * 64 + lane;
                 r[0] = make_float4(acck[0][0], acck[0][1], acck[0][2], acck[0][3]);
@@ -1420,7 +1425,7 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
             __syncthreads();
         }
 
-        if (q3 == 0 && kin) {
+        if (q3 == 0 && kin && 8 * g < D) {
             // part 0 + part 1 + ..., then lane holds d = 8 g .. + 8 of its key
             float ks[8], vs[8];
 #pragma unroll
@@ -1437,7 +1442,22 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
                 vs[0] += v0.x; vs[1] += v0.y; vs[2] += v0.z; vs[3] += v0.w;
                 vs[4] += v1.x; vs[5] += v1.y; vs[6] += v1.z; vs[7] += v1.w;
             }
-            const int64_t off = (((int64_t)n * a.H + h) * a.Sk + key) * DP + 8 * g;
+            const int64_t off = (((int64_t)n * a.H + h) * a.Sk + key) * D + 8 * g;
+            if constexpr (WIN) {
+                ks[0] += run[0].x; ks[1] += run[0].y; ks[2] += run[0].z; ks[3] += run[0].w;
+                ks[4] += run[1].x; ks[5] += run[1].y; ks[6] += run[1].z; ks[7] += run[1].w;
+                vs[0] += run[2].x; vs[1] += run[2].y; vs[2] += run[2].z; vs[3] += run[2].w;
+                vs[4] += run[3].x; vs[5] += run[3].y; vs[6] += run[3].z; vs[7] += run[3].w;
+                if (!a.wlast) {
+                    float* pk = a.dkv + off;
+                    float* pv = pk + (int64_t)a.N * a.H * a.Sk * D;
+                    *reinterpret_cast<float4*>(pk) = make_float4(ks[0], ks[1], ks[2], ks[3]);
+                    *reinterpret_cast<float4*>(pk + 4) = make_float4(ks[4], ks[5], ks[6], ks[7]);
+                    *reinterpret_cast<float4*>(pv) = make_float4(vs[0], vs[1], vs[2], vs[3]);
+                    *reinterpret_cast<float4*>(pv + 4) = make_float4(vs[4], vs[5], vs[6], vs[7]);
+                    continue;
+                }
+            }
             half8 ok, ov;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -1450,8 +1470,8 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
     }
 
     if constexpr (DBIAS) {
-        const int qtiles = a.SqA / 32;
-        float* dst = a.partial + (((int64_t)c * a.H + h) * a.kblocks + kblk) * a.SqA * 64 + klocal;
+        const int qtiles = a.SqA / 32 - wt0;
+        float* dst = a.partial + ((((int64_t)c * a.H + h) * a.kblocks + kblk) * a.SqA + 32 * wt0) * 64 + klocal;
 #pragma unroll
         for (int u = 0; u < TT; ++u) {
             const int ut = q3 * TT + u;
@@ -1462,12 +1482,7 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
     }
 }
 
-template __global__ void attn_bwd_dkdv_reg3_kernel<12, true>(BwdArgs);
-template __global__ void attn_bwd_dkdv_reg3_kernel<12, false>(BwdArgs);
-template __global__ void attn_bwd_dkdv_reg3_kernel<8, true>(BwdArgs);
-template __global__ void attn_bwd_dkdv_reg3_kernel<8, false>(BwdArgs);
-
-// With more than one query window: dk = fp16(scale * sum of the windows' dK sums), dv = fp16(sum
+// With more than one query window of the LDS-partial kernel: dk = fp16(scale * sum of the windows' dK sums), dv = fp16(sum
 // of their dV sums), each summed in window order, four elements per thread (D % 4 == 0).
 __global__ __launch_bounds__(256) void attn_bwd_dkdv_sum_kernel(BwdArgs a) {
     const int64_t plane = (int64_t)a.N * a.H * a.Sk * a.D;
@@ -1617,6 +1632,7 @@ static int cu_count(int device) {
 struct BwdPlan {
     int DP = 32;
     int QT = 0;  // query tiles of the register-partial dK/dV kernel (4, 8 or 12), 0: not used
+    int n12 = 0, n8 = 0;  // the register kernel's query windows: n12 of 12 tiles, then n8 of 8
     int QG = 1;  // query groups of the dK/dV kernel
     int kblocks = 0, chunk = 0, chunks = 0;
     int wtiles = 1, windows = 1;  // query windows of the dK/dV kernel
@@ -1636,14 +1652,11 @@ static size_t dkdv_stage_bytes(int DP, int QG) {
     return 0;
 }
 
-// The dK/dV kernel's shape depends only on the problem and the device, never on want_dbias, so
-// dk and dv are bit-identical with and without dbias.
-//
-// Its dBias partial stays in LDS for a whole chunk of rows: 64 keys x the queries of a query
+// The LDS-partial kernel's plan. Its dBias partial stays in LDS for a whole chunk of rows: 64 keys x the queries of a query
 // window, 8 KB per 32-query tile. Where all of Sq does not fit next to the Q/dO staging, the
 // queries are split into windows of equal tile counts (one more grid dimension); each window's
 // dK and dV sums then go to the workspace in fp32 and dkdv_sum_kernel adds them in window order.
-static BwdPlan plan_bwd(int device, int64_t N, int64_t H, int64_t Sq, int64_t Sk, int64_t D) {
+static BwdPlan plan_lds(int device, int64_t N, int64_t H, int64_t Sq, int64_t Sk, int64_t D) {
     BwdPlan p;
     p.DP = D <= 32 ? 32 : D <= 64 ? 64 : 96;
     p.SqA = (int)(((Sq + 31) / 32) * 32);
@@ -1654,38 +1667,6 @@ static BwdPlan plan_bwd(int device, int64_t N, int64_t H, int64_t Sq, int64_t Sk
     const size_t tile_bytes = (size_t)64 * 32 * sizeof(float);
     const int64_t qtiles = std::max<int64_t>((Sq + 31) / 32, 1);
     const int64_t Nr = std::max<int64_t>(N, 1);  // N == 0 plans one (empty) chunk
-    if (D == 32 && qtiles <= 12) {
-        // the register-partial kernels: one workgroup of eight (QT 4), sixteen (QT 8) or twelve (QT 12) waves
-        // per CU, one row per pass;
-        // chunks trade rounds of workgroups against dbias partials to write and sum (one
-        // partial weighs about H kblocks / 128 row passes)
-        p.QT = qtiles <= 4 ? 4 : qtiles <= 8 ? 8 : 12;
-        p.QG = 1;
-        p.wtiles = (int)qtiles;
-        p.windows = 1;
-        const int64_t slots = (int64_t)cu_count(device);
-        const int64_t cols = std::max<int64_t>(H * p.kblocks, 1);
-        int64_t best = 1;
-        double best_cost = 1e300;
-        for (int64_t ch = 1; ch <= Nr; ++ch) {
-            const int64_t rows = (Nr + ch - 1) / ch;
-            const int64_t real = (Nr + rows - 1) / rows;
-            const int64_t rounds = (real * cols + slots - 1) / slots;
-            const double cost = (double)rounds * rows + (double)real * cols / 128.0;
-            if (cost < best_cost) {
-                best_cost = cost;
-                best = real;
-            }
-        }
-        p.chunk = (int)((Nr + best - 1) / best);
-        p.chunks = (int)((N + p.chunk - 1) / p.chunk);
-        p.delta_bytes = round256((size_t)N * H * p.SqA * sizeof(float));
-        p.SqB = 32 * p.QT;
-        p.biast_bytes = round256((size_t)H * (p.SkA + 1) * p.SqB * sizeof(float));
-        p.partial_bytes = round256((size_t)p.chunks * H * p.kblocks * p.SqA * 64 * sizeof(float));
-        p.bfrag_bytes = round256((size_t)H * p.SqA * p.SkA * sizeof(half_t));
-        return p;
-    }
     // row groups of the dK/dV kernel: at most the query tiles of a window, which they walk from
     // staggered starts; the most row groups (waves per CU) first, then the fewest windows
     int qg_max = p.DP == 32 ? 4 : 2;
@@ -1745,8 +1726,73 @@ static BwdPlan plan_bwd(int device, int64_t N, int64_t H, int64_t Sq, int64_t Sk
     return p;
 }
 
+// The register-partial kernels' plan (D <= 32): one workgroup of eight (QT 4), sixteen (QT 8) or
+// twelve (QT 12) waves per CU, one row per pass. Past 12 tiles the queries go in windows of 12 and 8
+// tiles, as few windows as there can be and as few padded tiles as they allow (at most 3). Chunks
+// trade rounds of workgroups against dbias partials to write and sum (one partial weighs about H
+// kblocks / 128 row passes).
+static BwdPlan plan_reg(int device, int64_t N, int64_t H, int64_t Sq, int64_t Sk, int64_t D) {
+    BwdPlan p;
+    p.DP = D <= 32 ? 32 : D <= 64 ? 64 : 96;
+    p.SqA = (int)(((Sq + 31) / 32) * 32);
+    p.kblocks = (int)((Sk + 63) / 64);
+    p.SkA = p.kblocks * 64;
+    const int64_t qtiles = std::max<int64_t>((Sq + 31) / 32, 1);
+    const int64_t Nr = std::max<int64_t>(N, 1);  // N == 0 plans one (empty) chunk
+    p.QT = qtiles <= 4 ? 4 : qtiles <= 8 ? 8 : 12;
+    p.QG = 1;
+    p.wtiles = (int)qtiles;
+    p.windows = (int)((qtiles + 11) / 12);
+    if (p.windows > 1) {
+        p.n12 = (int)std::max<int64_t>((qtiles - 8 * p.windows + 3) / 4, 0);
+        p.n8 = p.windows - p.n12;
+    }
+    const int64_t slots = (int64_t)cu_count(device);
+    const int64_t cols = std::max<int64_t>(H * p.kblocks, 1);
+    int64_t best = 1;
+    double best_cost = 1e300;
+    for (int64_t ch = 1; ch <= Nr; ++ch) {
+        const int64_t rows = (Nr + ch - 1) / ch;
+        const int64_t real = (Nr + rows - 1) / rows;
+        const int64_t rounds = (real * cols + slots - 1) / slots;
+        const double cost = (double)rounds * rows + (double)real * cols / 128.0;
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = real;
+        }
+    }
+    p.chunk = (int)((Nr + best - 1) / best);
+    p.chunks = (int)((N + p.chunk - 1) / p.chunk);
+    p.delta_bytes = round256((size_t)N * H * p.SqA * sizeof(float));
+    p.SqB = 32 * (p.windows > 1 ? 12 * p.n12 + 8 * p.n8 : p.QT);
+    p.biast_bytes = round256((size_t)H * (p.SkA + 1) * p.SqB * sizeof(float));
+    p.partial_bytes = round256((size_t)p.chunks * H * p.kblocks * p.SqA * 64 * sizeof(float));
+    p.dkv_bytes = p.windows > 1 ? round256((size_t)2 * N * H * Sk * D * sizeof(float)) : 0;
+    p.bfrag_bytes = round256((size_t)H * p.SqA * p.SkA * sizeof(half_t));
+    return p;
+}
+
 static size_t bwd_workspace_bytes(const BwdPlan& p) {
     return 2 * p.delta_bytes + p.biast_bytes + p.partial_bytes + p.dkv_bytes + p.bfrag_bytes;
+}
+
+// The size of the static scratch of clk_attention_bwd_noalloc: enough for [512, 8, 384, 32], which
+// needs 86.3 MiB of query terms, transposed bias and dBias partials.
+constexpr size_t kNoAllocScratchBytes = size_t(96) << 20;
+
+static bool reg_only(int64_t Sq, int64_t D) { return D == 32 && Sq <= 384; }
+
+// The dK/dV kernel's shape depends only on the problem and the device, never on want_dbias or the
+// entry point, so dk and dv are bit-identical with and without dbias, and with either scratch.
+// D <= 32 takes the register kernels, which measured faster than the LDS-partial one at every size
+// ([640, 4, 640, 32]: 871 against 992 + 207 us; [1024, 8, 256, 8]: 319 against 358), unless
+// only the latter's scratch fits clk_attention_bwd_noalloc's.
+static BwdPlan plan_bwd(int device, int64_t N, int64_t H, int64_t Sq, int64_t Sk, int64_t D) {
+    if (D > 32) return plan_lds(device, N, H, Sq, Sk, D);
+    const BwdPlan r = plan_reg(device, N, H, Sq, Sk, D);
+    if (reg_only(Sq, D) || bwd_workspace_bytes(r) <= kNoAllocScratchBytes) return r;
+    const BwdPlan l = plan_lds(device, N, H, Sq, Sk, D);
+    return bwd_workspace_bytes(l) <= kNoAllocScratchBytes ? l : r;
 }
 
 template <int DP, int QG>
@@ -1785,28 +1831,44 @@ static int launch_bwd(hipStream_t stream, const BwdArgs& a, const BwdPlan& p, bo
     stage_mark(stream, 2);
     if (p.QT > 0) {
         if constexpr (DP == 32) {
-            const int64_t g2 = (int64_t)p.chunks * a.H * p.kblocks;
-#define CLK_DKDV_REG(QT_)                                                                        \
-    if (p.QT == QT_) {                                                                           \
-        if (want_dbias) {                                                                        \
-            hipLaunchKernelGGL((attn_bwd_dkdv_reg_kernel<QT_, true>), dim3((unsigned)g2), dim3(512), 0, stream, a); \
-        } else {                                                                                 \
-            hipLaunchKernelGGL((attn_bwd_dkdv_reg_kernel<QT_, false>), dim3((unsigned)g2), dim3(512), 0, stream, a); \
-        }                                                                                        \
+            const dim3 grid((unsigned)((int64_t)p.chunks * a.H * p.kblocks));
+#define CLK_DKDV(KERNEL_, THREADS_, ARGS_)                                                       \
+    if (want_dbias) {                                                                            \
+        hipLaunchKernelGGL((KERNEL_(true)), grid, dim3(THREADS_), 0, stream, ARGS_);             \
+    } else {                                                                                     \
+        hipLaunchKernelGGL((KERNEL_(false)), grid, dim3(THREADS_), 0, stream, ARGS_);            \
     }
-            CLK_DKDV_REG(4)
-#define CLK_DKDV_PARTS(QT_)                                                                      \
-    if (p.QT == QT_) {                                                                           \
-        constexpr int kNT = PartTile<QT_>::kThreads;                                             \
-        if (want_dbias) {                                                                        \
-            hipLaunchKernelGGL((attn_bwd_dkdv_reg3_kernel<QT_, true>), dim3((unsigned)g2), dim3(kNT), 0, stream, a); \
-        } else {                                                                                 \
-            hipLaunchKernelGGL((attn_bwd_dkdv_reg3_kernel<QT_, false>), dim3((unsigned)g2), dim3(kNT), 0, stream, a); \
-        }                                                                                        \
-    }
-            CLK_DKDV_PARTS(8) CLK_DKDV_PARTS(12)
-#undef CLK_DKDV_PARTS
-#undef CLK_DKDV_REG
+#define CLK_REG4(DB_) attn_bwd_dkdv_reg_kernel<4, DB_>
+#define CLK_REG8(DB_) attn_bwd_dkdv_reg3_kernel<8, DB_, false>
+#define CLK_REG12(DB_) attn_bwd_dkdv_reg3_kernel<12, DB_, false>
+#define CLK_WIN8(DB_) attn_bwd_dkdv_reg3_kernel<8, DB_, true>
+#define CLK_WIN12(DB_) attn_bwd_dkdv_reg3_kernel<12, DB_, true>
+            if (p.windows > 1) {
+                BwdArgs aw = a;
+                aw.wt0 = 0;
+                for (int w = 0; w < p.windows; ++w) {
+                    aw.wfirst = w == 0;
+                    aw.wlast = w == p.windows - 1;
+                    if (w < p.n12) {
+                        CLK_DKDV(CLK_WIN12, PartTile<12>::kThreads, aw)
+                    } else {
+                        CLK_DKDV(CLK_WIN8, PartTile<8>::kThreads, aw)
+                    }
+                    aw.wt0 += w < p.n12 ? 12 : 8;
+                }
+            } else if (p.QT == 4) {
+                CLK_DKDV(CLK_REG4, 512, a)
+            } else if (p.QT == 8) {
+                CLK_DKDV(CLK_REG8, PartTile<8>::kThreads, a)
+            } else {
+                CLK_DKDV(CLK_REG12, PartTile<12>::kThreads, a)
+            }
+#undef CLK_WIN12
+#undef CLK_WIN8
+#undef CLK_REG12
+#undef CLK_REG8
+#undef CLK_REG4
+#undef CLK_DKDV
         }
     } else if (p.QG == 4) {
         if constexpr (DP == 32) launch_dkdv<DP, 4>(stream, a, p, want_dbias);
@@ -1815,7 +1877,7 @@ static int launch_bwd(hipStream_t stream, const BwdArgs& a, const BwdPlan& p, bo
     } else {
         launch_dkdv<DP, 1>(stream, a, p, want_dbias);
     }
-    if (p.windows > 1) {
+    if (p.QT == 0 && p.windows > 1) {
         const int64_t n4 = (int64_t)a.N * a.H * a.Sk * a.D / 4;
         const int64_t gs = std::min<int64_t>((n4 + 255) / 256, 8192);
         hipLaunchKernelGGL(attn_bwd_dkdv_sum_kernel, dim3((unsigned)gs), dim3(256), 0, stream, a);
@@ -1855,14 +1917,10 @@ extern "C" int clk_attention_bwd_plan(int32_t device, int64_t N, int64_t H, int6
     if (plan == nullptr || count < 0) return invalid("attention_bwd_plan: no output array");
     const BwdPlan p = plan_bwd(device, N, H, Sq, Sk, D);
     const int64_t vals[] = {p.QG, p.chunk, p.chunks, (p.chunk + p.QG - 1) / p.QG, p.windows,
-                            p.QT > 0 ? 1 : 0};
+                            p.QT > 0 && p.windows == 1 ? 1 : 0};
     for (int i = 0; i < count && i < 6; ++i) plan[i] = vals[i];
     return ok();
 }
-
-// The size of the static scratch of clk_attention_bwd_noalloc: enough for BASELINE C3
-// ([512, 8, 384, 32]: 86.3 MiB of query terms, transposed bias and dBias partials).
-constexpr size_t kNoAllocScratchBytes = size_t(96) << 20;
 
 // The scratch of clk_attention_bwd_noalloc, one copy per GPU, held until the process ends. Host
 // code never uses this name as an address: scratch_address() asks the runtime for each device's
@@ -1938,8 +1996,11 @@ static int attention_bwd_impl(clk_stream stream, int32_t device, const clk_buffe
     if (N * H * Sq == 0 && N * H * Sk == 0 && H * Sq * Sk == 0) return ok();  // nothing to write
     const size_t need = bwd_workspace_bytes(p);
     if (noalloc) {
-        if (need > kNoAllocScratchBytes) {
-            return invalid("attention_bwd_noalloc: these shapes need " + std::to_string(need) +
+        // (the register windows need less than the LDS-partial kernel's; the shapes that this entry
+        // point takes are still those whose LDS-partial scratch fits)
+        const size_t ask = reg_only(Sq, D) ? need : std::max(need, bwd_workspace_bytes(plan_lds(device, N, H, Sq, Sk, D)));
+        if (ask > kNoAllocScratchBytes) {
+            return invalid("attention_bwd_noalloc: these shapes need " + std::to_string(ask) +
                            " bytes of scratch, the library's static scratch holds " +
                            std::to_string(kNoAllocScratchBytes));
         }
