@@ -1320,18 +1320,9 @@ void epilogue_kernel(EpiArgs a) {
 
 // ---- transition -------------------------------------------------------------------------------
 //
-// out^T = W2^T relu(W1 X^T + b1) + b2 over hidden chunks of 64: the first product's accumulator
-// (rows = hidden units in pair order) is exactly the B operand of the second, so the hidden
-// activation never leaves registers. At C = 128 and 256 the weights do not fit in LDS whole, so
-// 64-unit chunks stream through it (each through registers into one buffer between two barriers)
-// and every weight fragment a wave reads feeds one MFMA per 16-row block of its rows: at C = 128 a
-// 256-row tile (two blocks a wave, which halves the LDS weight reads per MFMA: the kernel is bound
-// by them), at C = 256 128 rows. The biases live in LDS, so no global load is waited for between a
-// chunk's prefetch and its use; the last chunk prefetches the first for the next tile. At C = 64
-// both weights fit in LDS, and transition_rows_kernel below serves that width.
-constexpr int kHid = 64;
-template <int C>
-constexpr int trans_rows() { return C == 128 ? 256 : 128; }
+// out^T = W2^T relu(W1 X^T + b1) + b2: the first product's accumulator (rows = hidden units in pair
+// order) is exactly the B operand of the second, so the hidden activation never leaves registers.
+constexpr int kHid = 64;  // hidden units per block of w2T
 
 struct TransArgs {
     const half_t* x;
@@ -1343,178 +1334,289 @@ struct TransArgs {
     float eps;
 };
 
+// The transition at C = 128 and 256, whose weights (128 KB to 1 MB) do not fit in LDS whole: chunks
+// of HC hidden units stream through two LDS buffers by direct-to-LDS loads, the next chunk's issued
+// at the start of a chunk and landed at its one closing barrier. A workgroup is WV waves of RB 16-row
+// blocks each; a wave holds its rows' LayerNorm output (the B operands, loaded and normalised in
+// registers as in transition_rows_kernel below) and its output accumulators for the whole tile, so
+// LDS carries nothing but weights and every 1 KB weight fragment read feeds RB products. LDS reads
+// bound the products: a fragment read takes the LDS for 4.6 to 8 cycles, in which the CU's four
+// SIMDs finish one to two 16x16x32 products. RB = 2 fills 256 registers at C = 256 (two waves per
+// SIMD); at C = 128, where 3 and 4 would fit, they measured no faster (M = 262144: 85 and 82 against
+// 81 us before the rows' own registers), which left room for the next tile's rows.
+// The hidden units go 32 at a time: two paired W1 blocks give the lane hidden units 32 p + 8 g .. +7
+// of its rows, which after relu and rounding to fp16 are its B operand of the second product's step
+// p. Both products start from their biases, and relu runs on the rounded fp16 pairs.
+// - Keep decisions come from a ballot of the keep values of the wave's keep unit (64 rows, 32 at C =
+//   256, cuda/volta_ops.cu:551-553, which holds all of its rows); a wave with nothing to compute
+//   keeps step with the barriers. Padding stores zeros; the stores of skipped rows and rows past M
+//   go to an offset past the tile's end, which the hardware drops.
+// Reading the fragments a group ahead of their products took 11% off, the rows' own registers another 8%
+// with add_input at C = 128. Against the kernel before (the row tile in LDS, weight chunks through
+// registers between two barriers; at C = 256 one wave per SIMD): C = 256, H = 1024, M = 127508: 331 ->
+// 140 us (0.96 PFLOP/s); C = 128, H = 512, M = 262144, bf16 with add_input: 102 -> 83 us (0.83 PFLOP/s).
+// At M = 262144 neither the matrix cores (27 us at their nominal rate, 56 at a large library product's)
+// nor LDS reads (27 us) bound it alone: the eight waves meet at a barrier per chunk.
 template <int C>
-struct TransTile {
-    static constexpr int KS = C / 32;
-    static constexpr int kW1 = 4 * KS * kWave * 8;        // halfs: 4 hidden blocks
-    static constexpr int kW2 = (C / 16) * 2 * kWave * 8;  // halfs: C/16 blocks x 2 steps
-    static constexpr int kChunks = (kW1 + kW2) / 8;
-    static constexpr int kCPT = kChunks / kFThreads;
-    static constexpr int kSub = C > 128 ? 32 : 64;        // keep granularity (volta_ops.cu:551-553)
-};
+constexpr int trans_chunk() { return C == 128 ? 128 : 64; }  // hidden units per chunk: 64 KB of weights
+constexpr size_t trans_lds_bytes(int C, int H) {
+    const int hc = C == 128 ? 128 : 64;
+    return (size_t)2 * 2 * hc * C * 2 + (size_t)(3 * C + H) * 4;
+}
 
-// Threads per workgroup (one workgroup per CU): at C = 128 eight waves of two 16-row blocks, at
-// C = 256 four waves of two row blocks.
-constexpr int trans_threads(int C) { return C <= 128 ? 512 : 256; }
-
-template <int C, bool ADD, int TH, bool BF>
-__global__ __launch_bounds__(TH, TH / 256) void transition_kernel(TransArgs a) {
-    using T = TransTile<C>;
-    constexpr int kTR = trans_rows<C>();
-    constexpr int TW = TH / kWave, RB = kTR / 16 / TW, kCPT = T::kChunks / TH;
-    static_assert(RB * TW * 16 == kTR && kCPT * TH == T::kChunks, "whole row blocks and chunks");
-    constexpr int KS = T::KS, NCB = C / 16, NSUB = kTR / T::kSub;
-    static_assert(C != 64, "C = 64 is transition_rows_kernel's");
-    extern __shared__ __attribute__((aligned(16))) half_t lds[];
-    half_t* Xf = lds;                   // the row tile's LayerNorm output, fragment-major
-    half_t* W1 = Xf + kTR * C;          // (C = 256) hidden chunk of w1, then of w2
-    half_t* W2 = W1 + T::kW1;
-    float* sc = reinterpret_cast<float*>(W2 + T::kW2);
-    float* of = sc + C;
-    float* b2s = of + C;
-    float* b1s = b2s + C;  // [H]
-    for (int i = threadIdx.x; i < C; i += TH) {
-        sc[i] = a.scale[i];
-        of[i] = a.offset[i];
-        b2s[i] = a.b2[i];
-    }
-    for (int i = threadIdx.x; i < a.H; i += TH) b1s[i] = a.b1[i];
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+template <int C, int RB, int WV, bool ADD, bool BF>
+__global__ __launch_bounds__(WV * kWave, 2) void transition_stream_kernel(TransArgs a) {
+    constexpr int KS = C / 32, NCB = C / 16, HC = trans_chunk<C>(), kRows = RB * 16, NG = RB == 1 ? 4 : 2;
+    constexpr int kUnit = C > 128 ? 32 : 64;           // keep granularity
+    constexpr int kF1 = HC / 16 * KS, kF2 = NCB * (HC / 32);  // 1 KB fragments of w1 and of w2 per chunk
+    static_assert(kRows <= kUnit && (kF1 + kF2) % WV == 0, "one keep unit per wave, whole fragments per wave");
+    constexpr uint32_t kDrop = 0x80000000u;  // a store offset past every tile's end
+    using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
+    // (two arrays, chosen at compile time: the compiler then knows that a chunk's reads do not alias
+    // the loads in flight)
+    __shared__ __attribute__((aligned(16))) half_t Wa[(kF1 + kF2) * 512];
+    __shared__ __attribute__((aligned(16))) half_t Wb[(kF1 + kF2) * 512];
+    __shared__ __attribute__((aligned(16))) float prm[3 * C + 4 * C];  // scale, offset, b2, b1
+    const float *sc = prm, *of = prm + C, *b2s = prm + 2 * C, *b1s = prm + 3 * C;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int r16 = lane & 15, g = lane >> 4;
-    const int wv = __builtin_amdgcn_readfirstlane(wave);
-    const int tiles = (a.M + kTR - 1) / kTR;
-    const int chunks = a.H / kHid;
+    const int tiles = (a.M + WV * kRows - 1) / (WV * kRows);
+    const int chunks = a.H / HC;  // even: H is 2 C or 4 C
+    const bool has_keep = a.keep != nullptr;
 
-    // weight chunk j: W1 fragments of hidden rows 64 j + pair_row(hb, r), W2 fragments of output
-    // channels pair_row(cb, r) over hidden 64 j + 32 kt + 8 g ..; fragment t (of 64 lanes' 16-byte
-    // operands) is 16-byte chunks 64 t .. + 63 of the chunk, and thread i stages chunk i
-    half8 wreg[kCPT];
-    const auto fetch_w = [&](int j) {
+    // chunk j into buffer buf: fragment t < kF1 is w1's (hidden block t / KS, step t % KS), then w2's
+    // (channel block, step of 32 hidden units); every wave loads (kF1 + kF2) / WV of them
+    const auto r1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.w1T), 0, (uint32_t)(a.H * C) * 2u, 0x00020000);
+    const auto r2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.w2T), 0, (uint32_t)(a.H * C) * 2u, 0x00020000);
+    const uint32_t o1 = (uint32_t)((8 * (r16 >> 2) + (r16 & 3)) * C + 8 * g) * 2u;
+    const uint32_t o2 = (uint32_t)((8 * (r16 >> 2) + (r16 & 3)) * kHid + 8 * g) * 2u;
+    const auto dma = [&](int j, half_t* buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < kCPT; ++u) {
-            const int i = threadIdx.x + u * TH;
-            const int l = i % kWave, t = i / kWave;
-            if (i < T::kW1 / 8) {
-                const int ks = t % KS, hb = t / KS;
-                const int hid = kHid * j + pair_row(hb, l & 15);
-                wreg[u] = fld8(a.w1T + (int64_t)hid * C + 32 * ks + 8 * (l >> 4));
+        for (int u = 0; u < (kF1 + kF2) / WV; ++u) {
+            const int t = u * WV + wave;  // kF1 is a multiple of WV: a load's matrix is known at compile time
+            if (u * WV < kF1) {
+                const int ks = t % KS, hb = t / KS;  // rows of w1T 32 (hb / 2) + 4 (hb % 2) + (lane's)
+                const uint32_t base = (uint32_t)((HC * j + 32 * (hb >> 1) + 4 * (hb & 1)) * C + 32 * ks) * 2u;
+                dma_lds<16>(r1, buf + 512 * t, o1 + base);
             } else {
-                const int t2 = t - T::kW1 / (8 * kWave);
-                const int kt = t2 & 1, cb = t2 >> 1;
-                const int c = pair_row(cb, l & 15);
-                wreg[u] = fld8(a.w2T + ((int64_t)j * C + c) * kHid + 32 * kt + 8 * (l >> 4));
+                const int t2 = t - kF1, kt = t2 % (HC / 32), cb = t2 / (HC / 32);
+                const int hj = HC * j / kHid + (kt >> 1);  // w2T's block of 64 hidden units
+                const uint32_t base = (uint32_t)((hj * C + 32 * (cb >> 1) + 4 * (cb & 1)) * kHid + 32 * (kt & 1)) * 2u;
+                dma_lds<16>(r2, buf + 512 * t, o2 + base);
             }
         }
     };
-    const auto store_w = [&]() {
+    static_assert(kF1 % WV == 0, "a load's matrix is known at compile time");
+
+    // this wave's rows of tile t (rows past M repeat row M - 1) and the keep value of row
+    // lane % kUnit of their keep unit
+    // Registers allow the next tile's rows a place of their own at C = 128 (kNext), fetched at the
+    // start of a tile, with the tile's raw rows kept for the residual. At C = 256 they are fetched
+    // after the last chunk into the operands' registers, with add_input after this tile's rows have
+    // come there once more for the residual (in the operands' own layout).
+    constexpr bool kNext = C == 128;
+    half8 xop[RB][KS], xn[kNext ? RB : 1][KS];
+    half_t kraw = (half_t)1.f;
+    const auto fetch_block = [&](int t, int rb, half8 (&x)[KS]) __attribute__((always_inline)) {
+        const half_t* px = a.x + (int64_t)min((t * WV + wave) * kRows + 16 * rb + r16, a.M - 1) * C + 8 * g;
 #pragma unroll
-        for (int u = 0; u < kCPT; ++u) fst8(W1 + (threadIdx.x + u * TH) * 8, wreg[u]);
+        for (int ks = 0; ks < KS; ++ks) x[ks] = fld8(px + 32 * ks);
+    };
+    const auto fetch = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) fetch_block(t, rb, kNext ? xn[kNext ? rb : 0] : xop[rb]);
+    };
+    const auto fetch_keep = [&](int t) __attribute__((always_inline)) {
+        const int u0 = ((t * WV + wave) * kRows) & ~(kUnit - 1);
+        if (has_keep) kraw = a.keep[min(u0 + (lane & (kUnit - 1)), a.M - 1)];
     };
 
-    RowTile<C, kTR, TH> xt;
-    fetch_w(0);
-    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const int m0 = tile * kTR;
-        int work[NSUB];
-        bool any = false;
+    int t = blockIdx.x;
+    dma(0, Wa);
+    fetch(t);
+    fetch_keep(t);
+    for (int i = threadIdx.x; i < C; i += WV * kWave) {
+        prm[i] = a.scale[i];
+        prm[C + i] = a.offset[i];
+        prm[2 * C + i] = (float)a.b2[i];
+    }
+    for (int i = threadIdx.x; i < a.H; i += WV * kWave) prm[3 * C + i] = (float)a.b1[i];
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    __syncthreads();
+
+    for (;;) {
+        const int m0 = (t * WV + wave) * kRows;
+        const float kv = (m0 & ~(kUnit - 1)) + (lane & (kUnit - 1)) < a.M ? (float)kraw : -1.f;
+        const bool any_live = __any(kv > 0.f), any_zero = __any(kv == 0.f);
+        const int work = any_live ? (int)kCompute : any_zero ? (int)kPadding : (int)kSkip;
+        half8 xr[kNext && ADD ? RB : 1][KS];  // the raw rows
+        if constexpr (kNext) {
 #pragma unroll
-        for (int s = 0; s < NSUB; ++s) {
-            work[s] = tile_work(a.keep, a.M, m0 + s * T::kSub, T::kSub, -1.f);
-            any |= work[s] == kCompute;
-        }
-        if (!any) {
-            if (!ADD) {
-                for (int i = threadIdx.x; i < kTR * C / 8; i += TH) {
-                    const int r = i / (C / 8), c = (i % (C / 8)) * 8;
-                    if (work[r / T::kSub] == kPadding && m0 + r < a.M)
-                        fst8(a.out + (int64_t)(m0 + r) * C + c, fzero8());
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    xop[rb][ks] = xn[kNext ? rb : 0][ks];
+                    if constexpr (ADD) xr[kNext && ADD ? rb : 0][ks] = xn[kNext ? rb : 0][ks];
                 }
-            }
-            continue;
         }
-        fetch_rows<C, kTR>(xt, a.x, a.M, m0);
-        __syncthreads();
-        ln_rows_to_frags<C, kTR, false, true, TH, BF>(Xf, xt, sc, of, a.eps);
-
-        float4v acc[NCB][RB];
-#pragma unroll
-        for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) acc[cb][rb] = float4v{0.f, 0.f, 0.f, 0.f};
-        half8 xop[RB][KS];
-        for (int j = 0; j < chunks; ++j) {
-            __syncthreads();  // the previous chunk's weight reads are done
-            store_w();
-            __syncthreads();
-            if (j == 0) {
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-                    for (int ks = 0; ks < KS; ++ks) xop[rb][ks] = fld8(Xf + frag(RB * wave + rb, ks, KS, lane));
-            }
-            fetch_w(j + 1 < chunks ? j + 1 : 0);  // the first chunk again for the next tile
-
-            // hidden^T for 64 units x this wave's 16 RB rows
-            float4v hacc[4][RB];
-#pragma unroll
-            for (int hb = 0; hb < 4; ++hb)
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb) hacc[hb][rb] = float4v{0.f, 0.f, 0.f, 0.f};
+        // LayerNorm of the wave's rows, in place: a row's statistics over its four lanes
+        const auto pin_rows = [&](int rb) __attribute__((always_inline)) {
+            typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-                for (int hb = 0; hb < 4; ++hb) {
-                    const half8 w = fld8(W1 + frag(hb, ks, KS, lane));
-#pragma unroll
-                    for (int rb = 0; rb < RB; ++rb) hacc[hb][rb] = mfma16x16x32(w, xop[rb][ks], hacc[hb][rb]);
-                }
+                u4 w = __builtin_bit_cast(u4, xop[rb][ks]);
+                asm volatile("" : "+v"(w));
+                xop[rb][ks] = __builtin_bit_cast(half8, w);
             }
-            half8 hop[2][RB];
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt) {
-                float b1v[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) b1v[e] = b1s[kHid * j + 32 * kt + 8 * g + e];
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        hop[kt][rb][e] = (half_t)fmaxf(hacc[2 * kt + (e >> 2)][rb][e & 3] + b1v[e], 0.f);
-            }
-#pragma unroll
-            for (int cb = 0; cb < NCB; ++cb) {
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt) {
-                    const half8 w = fld8(W2 + frag(cb, kt, 2, lane));
-#pragma unroll
-                    for (int rb = 0; rb < RB; ++rb) acc[cb][rb] = mfma16x16x32(w, hop[kt][rb], acc[cb][rb]);
-                }
-            }
-        }
-
-        // lane: channels 32 (cb/2) + 8 g .. +7 of rows m0 + 16 (RB wave + rb) + r16
+            __builtin_amdgcn_sched_barrier(0);
+        };
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            const int lr = 16 * (RB * wave + rb) + r16, row = m0 + lr;
-            const int w = work[lr / T::kSub];
-            if (row >= a.M || w == kSkip || (ADD && w == kPadding)) continue;
+            float s = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) s += act_get<BF>(xop[rb][ks], e);
+            s += __shfl_xor(s, 16);
+            s += __shfl_xor(s, 32);
+            const float mean = s * (1.f / C);
+            // (the raw values are converted anew in each pass: kept as fp32 they would spill)
+            pin_rows(rb);
+            float q = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float d = act_get<BF>(xop[rb][ks], e) - mean;
+                    q += d * d;
+                }
+            q += __shfl_xor(q, 16);
+            q += __shfl_xor(q, 32);
+            const float rstd = __builtin_amdgcn_rsqf(q * (1.f / C) + a.eps);
+            pin_rows(rb);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                half8 y;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int col = 32 * ks + 8 * g + e;
+                    y[e] = (half_t)((act_get<BF>(xop[rb][ks], e) - mean) * rstd * sc[col] + of[col]);
+                }
+                xop[rb][ks] = y;
+                __builtin_amdgcn_sched_barrier(0);  // (hoisting the parameters' reads would spill)
+            }
+            pin_rows(rb);
+        }
+        const int nt = t + gridDim.x, ft = min(nt, tiles - 1);
+        if constexpr (kNext) {
+            fetch(ft);
+            fetch_keep(ft);
+        }
+        // the output starts from b2: channel 32 (cb / 2) + 8 g + 4 (cb % 2) + i of row (rb, r16)
+        float4v acc[NCB][RB];
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) {
+            const float4v b = *reinterpret_cast<const float4v*>(b2s + 32 * (cb >> 1) + 8 * g + 4 * (cb & 1));
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) acc[cb][rb] = b;
+        }
+        // A chunk's products in the order of its fragments: for each 32 hidden units p, w1's 2 KS, then
+        // w2's NCB. They are read NG at a time, a group ahead of the products that use it (the
+        // scheduling barriers keep it so), in two register sets.
+        const auto chunk = [&](const half_t* W, const float* b1c) __attribute__((always_inline)) {
+            constexpr int kPer = 2 * KS + NCB, kGroups = (HC / 32) * kPer / NG;
+            static_assert((2 * KS) % NG == 0 && KS % NG == 0 && NCB % NG == 0, "groups do not straddle");
+            half8 wf[2][NG];
+            float4v hacc[RB], b1v;
+            half8 hop[RB];
+            const auto load = [&](int gi, half8 (&w)[NG]) __attribute__((always_inline)) {
+                const int p = gi * NG / kPer, f = gi * NG % kPer;
+#pragma unroll
+                for (int u = 0; u < NG; ++u)
+                    w[u] = fld8(f < 2 * KS ? W + frag(2 * p + (f + u) / KS, (f + u) % KS, KS, lane)
+                                           : W + kF1 * 512 + frag(f + u - 2 * KS, p, HC / 32, lane));
+                if (f < 2 * KS && f % KS == 0)
+                    b1v = *reinterpret_cast<const float4v*>(b1c + 32 * p + 8 * g + 4 * (f / KS));
+            };
+            load(0, wf[0]);
+#pragma unroll
+            for (int gi = 0; gi < kGroups; ++gi) {
+                const half8 (&w)[NG] = wf[gi & 1];
+                const int f = gi * NG % kPer;
+                if (f < 2 * KS && f % KS == 0) {
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) hacc[rb] = b1v;
+                }
+                if (gi + 1 < kGroups) load(gi + 1, wf[(gi + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (f < 2 * KS) {
+                    const int hb = f / KS, ks0 = f % KS;
+#pragma unroll
+                    for (int u = 0; u < NG; ++u)
+#pragma unroll
+                        for (int rb = 0; rb < RB; ++rb) hacc[rb] = mfma16x16x32(w[u], xop[rb][ks0 + u], hacc[rb]);
+                    if (ks0 + NG == KS) {
+#pragma unroll
+                        for (int rb = 0; rb < RB; ++rb) {
+                            half4 y;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) y[i] = (half_t)hacc[rb][i];
+                            y = __builtin_elementwise_max(y, half4{});
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) hop[rb][4 * hb + i] = y[i];
+                        }
+                    }
+                } else {
+                    const int cb0 = f - 2 * KS;
+#pragma unroll
+                    for (int u = 0; u < NG; ++u)
+#pragma unroll
+                        for (int rb = 0; rb < RB; ++rb) acc[cb0 + u][rb] = mfma16x16x32(w[u], hop[rb], acc[cb0 + u][rb]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        for (int j = 0; j < chunks; j += 2) {
+            dma(j + 1, Wb);
+            if (work == kCompute) chunk(Wa, b1s + HC * j);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            dma(j + 2 < chunks ? j + 2 : 0, Wa);  // the first chunk again for the next tile
+            if (work == kCompute) chunk(Wb, b1s + HC * (j + 1));
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+        }
+        if constexpr (!kNext) {
+            fetch(ADD ? t : ft);
+            fetch_keep(ft);
+        }
+        const int rows = max(min(kRows, a.M - m0), 0);
+        const auto ro = __builtin_amdgcn_make_buffer_rsrc(a.out + (int64_t)m0 * C, 0, (uint32_t)(rows * C) * 2u, 0x00020000);
+        const bool store = work == kCompute || (!ADD && work == kPadding);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
 #pragma unroll
             for (int cp = 0; cp < NCB / 2; ++cp) {
-                const int col = 32 * cp + 8 * g;
-                half_t* dst = a.out + (int64_t)row * C + col;
-                if (w == kPadding) {
-                    fst8(dst, fzero8());
-                    continue;
-                }
-                const half8 xa = ADD ? fld8(a.x + (int64_t)row * C + col) : fzero8();
+                const uint32_t off = (uint32_t)((16 * rb + r16) * C + 32 * cp + 8 * g) * 2u;
                 half8 o;
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    o[e] = act_cvt<BF>(acc[2 * cp + (e >> 2)][rb][e & 3] + b2s[col + e] + act_get<BF>(xa, e));
-                fst8(dst, o);
+                for (int e = 0; e < 8; ++e) {
+                    const float res = !ADD ? 0.f : act_get<BF>(kNext ? xr[kNext && ADD ? rb : 0][cp] : xop[rb][cp], e);
+                    o[e] = act_cvt<BF>(ADD ? acc[2 * cp + (e >> 2)][rb][e & 3] + res : acc[2 * cp + (e >> 2)][rb][e & 3]);
+                }
+                if (!ADD && work == kPadding) o = fzero8();
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), ro, store ? off : kDrop, 0, 0);
+            }
+            if constexpr (ADD && !kNext) {
+                __builtin_amdgcn_sched_barrier(0);
+                fetch_block(ft, rb, xop[rb]);
             }
         }
+        if (nt >= tiles) break;
+        t = nt;
     }
+    // the chunk loaded for a next tile that does not come has landed: the loop's last wait covers it
 }
 
 // The transition at C = 64, where both weights fit in LDS at once (W1 [H][64] and W2 [64][H], at
@@ -1539,7 +1641,7 @@ constexpr size_t trans_rows_lds_bytes(int C, int H) { return (size_t)2 * H * C *
 template <bool ADD, bool BF>
 __global__ __launch_bounds__(kTransRowsThreads, 4) void transition_rows_kernel(TransArgs a) {
     constexpr int C = 64, KS = C / 32, NCB = C / 16, RB = kTransRowsTile / 16, TW = kTransRowsThreads / kWave;
-    constexpr int kKeep = TransTile<C>::kSub;
+    constexpr int kKeep = 64;
     constexpr uint32_t kDrop = 0x80000000u;  // a store offset past every tile's end
     using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
     extern __shared__ __attribute__((aligned(16))) half_t lds[];
@@ -2084,15 +2186,20 @@ static int run_transition_rows(const TransArgs& a, hipStream_t s) {
     return launch_status("transition");
 }
 
+template <int C, int RB, int WV, bool ADD, bool BF>
+static int run_transition_stream(const TransArgs& a, hipStream_t s) {
+    const int64_t tiles = ((int64_t)a.M + WV * RB * 16 - 1) / (WV * RB * 16);
+    const dim3 grid((unsigned)std::min<int64_t>(tiles, fused_cu_count()));
+    stage_mark(s, 0);
+    hipLaunchKernelGGL((transition_stream_kernel<C, RB, WV, ADD, BF>), grid, dim3(WV * kWave), 0, s, a);
+    stage_mark(s, 1);
+    return launch_status("transition");
+}
+
 template <int C, bool ADD, bool BF>
 static int run_transition(const TransArgs& a, hipStream_t s) {
     const int limit = fused_lds_limit();
-    // C = 64: both weights resident in LDS (at most 66 KB at H = 4C); wider: the row tile, one
-    // weight chunk, the LayerNorm parameters and the biases
-    using T = TransTile<C>;
-    constexpr int kTR = trans_rows<C>();
-    const size_t lds = C == 64 ? trans_rows_lds_bytes(64, a.H)
-                               : (size_t)kTR * C * 2 + (size_t)(T::kW1 + T::kW2) * 2 + (size_t)(3 * C + a.H) * 4;
+    const size_t lds = C == 64 ? trans_rows_lds_bytes(64, a.H) : trans_lds_bytes(C, 4 * C);
     if (limit > 0 && lds > (size_t)limit) {
         return invalid("transition: needs " + std::to_string(lds / 1024) + " KB shared, device allows " +
                        std::to_string(limit / 1024) + " KB");
@@ -2100,14 +2207,11 @@ static int run_transition(const TransArgs& a, hipStream_t s) {
     if constexpr (C == 64) {
         return run_transition_rows<ADD, BF>(a, s);
     } else {
-        constexpr int TH = trans_threads(C);
-        const int64_t tiles = (a.M + kTR - 1) / kTR;
-        const dim3 grid(persistent_grid(tiles, lds, 1));
-        if (int st = launch_fused("transition", transition_kernel<C, ADD, TH, BF>, grid, lds, s, &a, 0)) return st;
-        stage_mark(s, 0);
-        hipLaunchKernelGGL((transition_kernel<C, ADD, TH, BF>), grid, dim3(TH), lds, s, a);
-        stage_mark(s, 1);
-        return launch_status("transition");
+        // 128-row tiles where one round of them covers M, 256-row tiles past that: a round of 256-row
+        // tiles takes 59 us at C = 256, H = 4 C (21 at C = 128), one of 128-row tiles 43 (18), whose
+        // fragment reads feed one product each
+        if (a.M <= 128 * fused_cu_count()) return run_transition_stream<C, 1, 8, ADD, BF>(a, s);
+        return run_transition_stream<C, 2, 8, ADD, BF>(a, s);
     }
 }
 
