@@ -21,6 +21,7 @@ FFI's InvalidArgument) and a launch failure KernelError (Internal), with the lib
 There is no CPU fallback: without the built library every call raises.
 """
 import ctypes
+import struct
 
 import torch
 
@@ -47,7 +48,7 @@ class Buffer(ctypes.Structure):
                 ("dims", ctypes.POINTER(ctypes.c_int64))]
 
 
-_P = ctypes.POINTER(Buffer)
+_P = ctypes.c_void_p  # a Buffer by reference (byref), or its address
 _lib = None
 
 _SIGNATURES = {
@@ -114,6 +115,47 @@ def _ref(b):
     return ctypes.byref(b)
 
 
+# The same descriptions for a whole call, as the calls below pass them: packed at once into one array,
+# with the dimension arrays of shapes met before reused (they depend on the shape alone). A call of
+# eight tensors spent 18 us in buffer(), half of it on the dimension arrays, where the smallest
+# kernels take 5 us.
+_PACKED = [struct.Struct("<" + "QiiQ" * n) for n in range(16)]
+_FRAMES = [ctypes.c_char * (24 * n) for n in range(16)]
+assert ctypes.sizeof(Buffer) == 24
+_DIMS = {}
+_DIMS_MAX = 4096
+
+
+def _dims(shape):
+    if len(_DIMS) >= _DIMS_MAX:
+        _DIMS.clear()  # calls in flight hold the arrays they use
+    arr = (ctypes.c_int64 * max(len(shape), 1))(*shape)
+    d = _DIMS[shape] = (ctypes.addressof(arr), arr)
+    return d
+
+
+def _frame(*tensors):
+    """The addresses of the clk_buffers of `tensors`, and what the caller keeps until its call is
+    over; the tensors' checks are buffer()'s."""
+    vals, keep = [], []
+    for t in tensors:
+        code = _DTYPES.get(t.dtype)
+        if code is None:
+            raise TypeError("unsupported dtype %s" % t.dtype)
+        if not t.is_contiguous():
+            raise ValueError("tensors must be contiguous")
+        shape = t.shape
+        d = _DIMS.get(shape) or _dims(shape)
+        keep.append(d)
+        vals += (t.data_ptr(), code, len(shape), d[0])
+    n = len(tensors)
+    frame = _FRAMES[n]()
+    _PACKED[n].pack_into(frame, 0, *vals)
+    keep.append(frame)
+    base = ctypes.addressof(frame)
+    return range(base, base + 24 * n, 24), keep
+
+
 def _check(status):
     if status != 0:
         msg = lib().clk_last_error().decode()
@@ -123,6 +165,8 @@ def _check(status):
 
 
 def _stream(t):
+    if t.is_cuda:
+        return torch._C._cuda_getCurrentRawStream(t.device.index)
     return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
 
 
@@ -149,8 +193,8 @@ def attention_fwd(q, k, v, bias, kmask, scale, block_q=64, block_k=32, want_lse=
     if lse is None:
         lse = (torch.empty((n, h, sq), dtype=torch.float32, device=q.device) if want_lse
                else torch.zeros(1, dtype=torch.float32, device=q.device))
-    bufs = [buffer(t) for t in (q, k, v, bias, kmask, out, lse)]
-    _check(lib().clk_attention_fwd(_stream(q), q.device.index, *map(_ref, bufs), float(scale),
+    bufs, hold = _frame(q, k, v, bias, kmask, out, lse)
+    _check(lib().clk_attention_fwd(_stream(q), q.device.index, *bufs, float(scale),
                                    int(block_q), int(block_k), int(bool(want_lse))))
     return out, lse
 
@@ -161,19 +205,19 @@ def attention_packed(p, bias, kmask, gate_bias, scale, block_q=64, block_k=32, c
     x, y, _, h, d = p.shape
     out = torch.empty((x, y, h, d), dtype=torch.float16, device=p.device) if out is None else out
     if lims is None:
-        bufs = [buffer(t) for t in (p, bias, kmask, gate_bias, out)]
+        bufs, hold = _frame(p, bias, kmask, gate_bias, out)
         fn = lib().clk_attention_packed
     else:
-        bufs = [buffer(t) for t in (p, bias, kmask, gate_bias, lims, out)]
+        bufs, hold = _frame(p, bias, kmask, gate_bias, lims, out)
         fn = lib().clk_attention_packed_trim
-    _check(fn(_stream(p), p.device.index, *map(_ref, bufs), float(scale), int(block_q),
+    _check(fn(_stream(p), p.device.index, *bufs, float(scale), int(block_q),
               int(block_k), int(bool(column))))
     return out
 
 
 def attention_bwd_workspace(q, k):
-    return int(lib().clk_attention_bwd_workspace_size(q.device.index, _ref(buffer(q)),
-                                                      _ref(buffer(k))))
+    bufs, hold = _frame(q, k)
+    return int(lib().clk_attention_bwd_workspace_size(q.device.index, *bufs))
 
 
 def attention_bwd_plan(n, h, sq, sk, d, device=0):
@@ -195,8 +239,8 @@ def attention_bwd(q, k, v, bias, kmask, out, dout, lse, scale, want_dbias=True, 
     if workspace is None:
         need = attention_bwd_workspace(q, k)
         workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
-    bufs = [buffer(t) for t in (q, k, v, bias, kmask, out, dout, lse, dq, dk, dv, dbias)]
-    _check(lib().clk_attention_bwd(_stream(q), q.device.index, *map(_ref, bufs), float(scale),
+    bufs, hold = _frame(q, k, v, bias, kmask, out, dout, lse, dq, dk, dv, dbias)
+    _check(lib().clk_attention_bwd(_stream(q), q.device.index, *bufs, float(scale),
                                    int(bool(want_dbias)), ctypes.c_void_p(workspace.data_ptr()),
                                    workspace.numel()))
     return dq, dk, dv, dbias
@@ -211,8 +255,8 @@ def attention_bwd_noalloc(q, k, v, bias, kmask, out, dout, lse, scale, want_dbia
         dbias = torch.empty(bias.shape, dtype=torch.float32, device=q.device)
     else:
         dq, dk, dv, dbias = grads
-    bufs = [buffer(t) for t in (q, k, v, bias, kmask, out, dout, lse, dq, dk, dv, dbias)]
-    _check(lib().clk_attention_bwd_noalloc(_stream(q), q.device.index, *map(_ref, bufs),
+    bufs, hold = _frame(q, k, v, bias, kmask, out, dout, lse, dq, dk, dv, dbias)
+    _check(lib().clk_attention_bwd_noalloc(_stream(q), q.device.index, *bufs,
                                            float(scale), int(bool(want_dbias))))
     return dq, dk, dv, dbias
 
@@ -220,10 +264,10 @@ def attention_bwd_noalloc(q, k, v, bias, kmask, out, dout, lse, scale, want_dbia
 def ln_gdp(x, scale, offset, wpT, bp, wgT, bg, mask, eps=1e-5):
     """VoltaLnGdp: left, right [P/2, M] F16, channel major."""
     m, p = x.shape[0], wpT.shape[0]
-    left = torch.empty((p // 2, m), dtype=x.dtype, device=x.device)
-    right = torch.empty((p // 2, m), dtype=x.dtype, device=x.device)
-    bufs = [buffer(t) for t in (x, scale, offset, wpT, bp, wgT, bg, mask, left, right)]
-    _check(lib().clk_ln_gdp(_stream(x), *map(_ref, bufs), float(eps)))
+    left = x.new_empty((p // 2, m))
+    right = x.new_empty((p // 2, m))
+    bufs, hold = _frame(x, scale, offset, wpT, bp, wgT, bg, mask, left, right)
+    _check(lib().clk_ln_gdp(_stream(x), *bufs, float(eps)))
     return left, right
 
 
@@ -231,12 +275,11 @@ def trimul_epilogue(x_cm, x, in_scale, in_offset, ln_scale, ln_offset, woT, bo, 
                     keep=None, eps=1e-5, add_input=False, out=None):
     """VoltaTrimulEpilogue: out [M,O] F16. out may be x itself with add_input."""
     m, o = x.shape[0], woT.shape[0]
-    out = torch.empty((m, o), dtype=x.dtype, device=x.device) if out is None else out
+    out = x.new_empty((m, o)) if out is None else out
     has_keep = keep is not None
     keep = keep if has_keep else _one(x, torch.float16)
-    bufs = [buffer(t) for t in (x_cm, x, in_scale, in_offset, ln_scale, ln_offset, woT, bo, wgT,
-                                bg, keep, out)]
-    _check(lib().clk_trimul_epilogue(_stream(x), *map(_ref, bufs), float(eps),
+    bufs, hold = _frame(x_cm, x, in_scale, in_offset, ln_scale, ln_offset, woT, bo, wgT, bg, keep, out)
+    _check(lib().clk_trimul_epilogue(_stream(x), *bufs, float(eps),
                                      int(bool(add_input)), int(has_keep)))
     return out
 
@@ -247,15 +290,15 @@ def ln_projection(x, scale, offset, wT=None, wbT=None, keep=None, eps=1e-5):
     m = x.shape[0]
     n = 0 if wT is None else wT.shape[0]
     heads = 0 if wbT is None else wbT.shape[0]
-    p = torch.empty((m, n), dtype=x.dtype, device=x.device) if n else _one(x, x.dtype)
-    bias = (torch.empty((heads, m), dtype=x.dtype, device=x.device) if heads
+    p = x.new_empty((m, n)) if n else _one(x, x.dtype)
+    bias = (x.new_empty((heads, m)) if heads
             else _one(x, x.dtype))
     has_keep = keep is not None
     keep = keep if has_keep else _one(x, torch.float16)
     wT = wT if n else _one(x, torch.float16)
     wbT = wbT if heads else _one(x, torch.float16)
-    bufs = [buffer(t) for t in (x, scale, offset, wT, wbT, keep, p, bias)]
-    _check(lib().clk_ln_projection(_stream(x), *map(_ref, bufs), float(eps), n, heads,
+    bufs, hold = _frame(x, scale, offset, wT, wbT, keep, p, bias)
+    _check(lib().clk_ln_projection(_stream(x), *bufs, float(eps), n, heads,
                                    int(has_keep)))
     return (p if n else None), (bias if heads else None)
 
@@ -263,13 +306,13 @@ def ln_projection(x, scale, offset, wT=None, wbT=None, keep=None, eps=1e-5):
 def output_projection(o, wT, b, residual=None, keep=None, out=None):
     """VoltaOutProj: out [M,N] = o@w + b [+ residual]; out may be residual itself."""
     m, n = o.shape[0], wT.shape[0]
-    out = torch.empty((m, n), dtype=o.dtype, device=o.device) if out is None else out
+    out = o.new_empty((m, n)) if out is None else out
     has_residual = residual is not None
     residual = residual if has_residual else _one(o, o.dtype)
     has_keep = keep is not None
     keep = keep if has_keep else _one(o, torch.float16)
-    bufs = [buffer(t) for t in (o, wT, b, residual, keep, out)]
-    _check(lib().clk_output_projection(_stream(o), *map(_ref, bufs), int(has_residual),
+    bufs, hold = _frame(o, wT, b, residual, keep, out)
+    _check(lib().clk_output_projection(_stream(o), *bufs, int(has_residual),
                                        int(has_keep)))
     return out
 
@@ -281,8 +324,8 @@ def transition(x, scale, offset, w1T, b1, w2T, b2, keep=None, eps=1e-5, add_inpu
     out = torch.empty_like(x) if out is None else out
     has_keep = keep is not None
     keep = keep if has_keep else _one(x, torch.float16)
-    bufs = [buffer(t) for t in (x, scale, offset, w1T, b1, w2T, b2, keep, out)]
-    _check(lib().clk_transition(_stream(x), *map(_ref, bufs), float(eps), int(bool(add_input)),
+    bufs, hold = _frame(x, scale, offset, w1T, b1, w2T, b2, keep, out)
+    _check(lib().clk_transition(_stream(x), *bufs, float(eps), int(bool(add_input)),
                                 int(has_keep)))
     return out
 
@@ -290,8 +333,8 @@ def transition(x, scale, offset, w1T, b1, w2T, b2, keep=None, eps=1e-5, add_inpu
 def layer_norm(x, scale, offset, eps=1e-5, out=None):
     """VoltaLayerNorm: out [M,C] F16, one-pass fp32 statistics."""
     out = torch.empty_like(x) if out is None else out
-    bufs = [buffer(t) for t in (x, scale, offset, out)]
-    _check(lib().clk_layer_norm(_stream(x), *map(_ref, bufs), float(eps)))
+    bufs, hold = _frame(x, scale, offset, out)
+    _check(lib().clk_layer_norm(_stream(x), *bufs, float(eps)))
     return out
 
 
@@ -300,8 +343,8 @@ def gated_dual_proj(x, wp, bp, wg, bg, mask, activation=0, out=None):
     activation 0 sigmoid, 1 swish."""
     m, n = x.shape[0], wp.shape[1]
     out = torch.empty((m, n), dtype=torch.float16, device=x.device) if out is None else out
-    bufs = [buffer(t) for t in (x, wp, bp, wg, bg, mask, out)]
-    _check(lib().clk_gated_dual_proj(_stream(x), x.device.index, *map(_ref, bufs), int(activation)))
+    bufs, hold = _frame(x, wp, bp, wg, bg, mask, out)
+    _check(lib().clk_gated_dual_proj(_stream(x), x.device.index, *bufs, int(activation)))
     return out
 
 
@@ -311,8 +354,8 @@ def opm_update(lhs, t, bias, norm, residual=None, eps=1e-3, out=None):
     b, (d, f) = lhs.shape[0], t.shape[1:]
     out = torch.empty((b, d, f), dtype=torch.float16, device=lhs.device) if out is None else out
     res = residual if residual is not None else _one(lhs, torch.float16)
-    bufs = [buffer(x) for x in (lhs, t, bias, norm, res, out)]
-    _check(lib().clk_opm_update(_stream(lhs), *map(_ref, bufs), float(eps), int(residual is not None)))
+    bufs, hold = _frame(lhs, t, bias, norm, res, out)
+    _check(lib().clk_opm_update(_stream(lhs), *bufs, float(eps), int(residual is not None)))
     return out
 
 
@@ -321,6 +364,6 @@ def opm_outer(left, right, wT, out=None):
     left [16,B,C], right [16,D,32], wT [F, 32 C], all fp16."""
     b, d, f = left.shape[1], right.shape[1], wT.shape[0]
     out = torch.empty((b, d, f), dtype=torch.float16, device=left.device) if out is None else out
-    bufs = [buffer(x) for x in (left, right, wT, out)]
-    _check(lib().clk_opm_outer(_stream(left), *map(_ref, bufs)))
+    bufs, hold = _frame(left, right, wT, out)
+    _check(lib().clk_opm_outer(_stream(left), *bufs))
     return out

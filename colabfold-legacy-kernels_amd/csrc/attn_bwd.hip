@@ -1652,6 +1652,14 @@ static size_t dkdv_stage_bytes(int DP, int QG) {
     return 0;
 }
 
+// The next count of chunks after `ch` that changes the rows per chunk, ceil(N / ch): the plans below
+// depend on ch through it alone, and look at about 2 sqrt(N) counts instead of N (a call plans up to
+// twice, and at N = 1024 the divisions took 20 us of host time each).
+static int64_t next_chunks(int64_t N, int64_t ch) {
+    const int64_t rows = (N + ch - 1) / ch;
+    return rows <= 1 ? N + 1 : (N - 1) / (rows - 1) + 1;
+}
+
 // The LDS-partial kernel's plan. Its dBias partial stays in LDS for a whole chunk of rows: 64 keys x the queries of a query
 // window, 8 KB per 32-query tile. Where all of Sq does not fit next to the Q/dO staging, the
 // queries are split into windows of equal tile counts (one more grid dimension); each window's
@@ -1701,7 +1709,7 @@ static BwdPlan plan_lds(int device, int64_t N, int64_t H, int64_t Sq, int64_t Sk
     const int64_t slots = (int64_t)cu_count(device) * per_cu;
     const int64_t cols = std::max<int64_t>(H * p.kblocks * p.windows, 1);
     int64_t best = 1, best_cost = INT64_MAX;
-    for (int64_t ch = 1; ch <= Nr; ++ch) {
+    for (int64_t ch = 1; ch <= Nr; ch = next_chunks(Nr, ch)) {
         // rows per workgroup, a whole number of passes of its QG row groups where N allows
         const int64_t rows = std::min<int64_t>(((Nr + ch - 1) / ch + p.QG - 1) / p.QG * p.QG, Nr);
         const int64_t real = (Nr + rows - 1) / rows;
@@ -1751,7 +1759,7 @@ static BwdPlan plan_reg(int device, int64_t N, int64_t H, int64_t Sq, int64_t Sk
     const int64_t cols = std::max<int64_t>(H * p.kblocks, 1);
     int64_t best = 1;
     double best_cost = 1e300;
-    for (int64_t ch = 1; ch <= Nr; ++ch) {
+    for (int64_t ch = 1; ch <= Nr; ch = next_chunks(Nr, ch)) {
         const int64_t rows = (Nr + ch - 1) / ch;
         const int64_t real = (Nr + rows - 1) / rows;
         const int64_t rounds = (real * cols + slots - 1) / slots;
