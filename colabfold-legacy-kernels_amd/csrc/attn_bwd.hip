@@ -422,6 +422,20 @@ __global__ __launch_bounds__(DqTile<DP>::kThreads, DP == 32 ? 4 : 1) void attn_b
         __builtin_amdgcn_s_waitcnt(kWaitVm0);
         __syncthreads();
     }
+    // a wave whose queries all lie past Sq only stages its share of the key tiles
+    if (wq >= a.Sq) {
+        for (int k0 = 0, buf = 0; k0 < a.Sk; k0 += T::kBK, buf ^= 1) {
+            const uint64_t keep_next = __ballot(mbyte != 0u);
+            if (k0 + T::kBK < a.Sk) {
+                fetch_kv(k0 + T::kBK, buf ^ 1, keep_next);
+                mbyte = fetch_mask(min(k0 + 2 * T::kBK, k_last));
+                if constexpr (DP != 32) stage(buf ^ 1, keep_next);
+            }
+            __builtin_amdgcn_s_waitcnt(kWaitVm0);
+            __syncthreads();
+        }
+        return;
+    }
     for (int k0 = 0; k0 < a.Sk; k0 += 2 * T::kBK) {
         tile(k0, 0, biasA, biasB);
         if (k0 + T::kBK < a.Sk) tile(k0 + T::kBK, 1, biasB, biasA);
