@@ -13,6 +13,8 @@
 //               are e in pair order, so that the accumulator, rounded to fp16, is already the B
 //               operand (k-slots e) of out^T[f, b] += W_c^T G_c^T, a 16x16x32 MFMA against the
 //               channel's weight rows staged in LDS. The [B, C E, D] product is never formed.
+#include <algorithm>
+
 #include "clk_common.h"
 
 namespace clk {
@@ -125,6 +127,159 @@ __global__ __launch_bounds__(256) void opm_update_kernel(OpmUpdateArgs a) {
         for (int j = 0; j < 8; ++j) h[j] = (half_t)((acc[j >> 2][i][j & 3] + bv[j]) / den[i] + (float)res[i][j]);
         *reinterpret_cast<half8*>(a.out + (int64_t)b * N + n) = h;
     }
+}
+
+// The same for K = 128, 256 and 512, with t^T in registers: a wave takes 32 columns, whose t^T operand
+// (2 x KS 16-byte registers) it forms once, through LDS by direct-to-LDS loads and transpose reads,
+// and then walks the rows b in blocks of 16, whose lhs rows stream fragment-major through four LDS
+// buffers, three blocks ahead. So t comes from HBM once and no row block waits for it again, a row
+// block's operand read feeds both of the wave's column blocks, and a row block costs one barrier; the
+// tiled kernel above stages every K step of both operands between two barriers.
+// The rows are split over workgroups that share a column tile (and t through L2) until those fill the
+// places for them.
+// The residual and norm of a row block are loaded with its lhs rows (loads complete in issue order, so
+// a later load of theirs would be waited for with everything before it).
+// K = 512, F = 128 (us, the tiled kernel's time first): B = D = 509 98.5 -> 71.6, 384 62 -> 53, 256 25.2 ->
+// 23.8; B = D = 128, where a workgroup would walk two blocks, 10.3 -> 12.9 and stays with the tiled kernel.
+template <int KS>
+__global__ __launch_bounds__(256, 2) void opm_update_cols_kernel(OpmUpdateArgs a, int splits, int blocks_per) {
+    constexpr int K = 32 * KS, kCh = K / 64;  // 64-row chunks of t, 16 KB of a workgroup's columns each
+    using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
+    constexpr uint32_t kDrop = 0x80000000u;
+    // lhs rows of a row block, fragment-major (at most 16 KB); before that, chunks of t
+    __shared__ __attribute__((aligned(16))) half_t X0[8192], X1[8192], T0[8192], T1[8192];
+    const int64_t N = (int64_t)a.D * a.F;
+    const int item = xcd_item(blockIdx.x, gridDim.x);
+    const int nt = item / splits, sp = item - nt * splits;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int r16 = lane & 15, g = lane >> 4;
+    const int64_t c0 = (int64_t)nt * 128;
+
+    // t rows 64 c .. + 63 of the workgroup's columns, rows of 256 bytes: load u of wave w brings rows
+    // 16 w + 4 u .. + 3, position p of row R holding its 16-byte chunk p ^ 4 (R % 4) (so the transpose
+    // reads' rows fall on different banks); columns past N read zeros
+    const auto dma_t = [&](int c, half_t* dst) __attribute__((always_inline)) {
+        const auto rt = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.t) + (int64_t)64 * c * N, 0,
+                                                          (uint32_t)(64 * N * 2), 0x00020000);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int R = 16 * wave + 4 * u + (lane >> 4), ch = (lane & 15) ^ (4 * (R & 3));
+            const int64_t col = c0 + 8 * ch;
+            dma_lds<16>(rt, dst + 512 * (4 * wave + u), col < N ? (uint32_t)((R * N + col) * 2) : kDrop);
+        }
+    };
+    half8 tw[2][KS];
+    const auto read_t = [&](int c, const half_t* src) __attribute__((always_inline)) {
+        const int j = r16 >> 2, q = r16 & 3;
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+            for (int hb = 0; hb < 2; ++hb) {
+                const int Rl = 32 * s2 + 8 * g + j, Rh = Rl + 4, ch = 4 * wave + q;
+                const half4 lo = lds_read_tr16(src + 128 * Rl + 8 * (ch ^ (4 * (Rl & 3))) + 4 * hb);
+                const half4 hi = lds_read_tr16(src + 128 * Rh + 8 * (ch ^ (4 * (Rh & 3))) + 4 * hb);
+                tw[hb][2 * c + s2] = half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            }
+    };
+    const auto buf_t = [&](int c) -> half_t* { return (c & 3) == 0 ? X0 : (c & 3) == 1 ? X1 : (c & 3) == 2 ? T0 : T1; };
+#pragma unroll
+    for (int c = 0; c < kCh && c < 4; ++c) dma_t(c, buf_t(c));
+
+    // epilogue operands: lane holds out[b][n .. n + 7] of its row b, one d (F is a multiple of 16)
+    const int64_t n = c0 + 32 * wave + 8 * g;
+    const bool nin = n < N;
+    const int64_t nc = nin ? n : N - 8;
+    const int d = (int)(nc / a.F), f = (int)(nc - (int64_t)d * a.F);
+    float bv[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bv[j] = a.bias[f + j];
+    const int blocks = (a.B + 15) / 16;
+    const int m_begin = sp * blocks_per, m_end = min(blocks, m_begin + blocks_per);
+
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < kCh && c < 4; ++c) read_t(c, buf_t(c));
+    if constexpr (kCh > 4) {
+        __syncthreads();
+#pragma unroll
+        for (int c = 4; c < kCh; ++c) dma_t(c, buf_t(c));
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+#pragma unroll
+        for (int c = 4; c < kCh; ++c) read_t(c, buf_t(c));
+    }
+    __syncthreads();
+
+    // lhs rows of row block m: fragment ks is lane (row r16, k 32 ks + 8 g ..); wave w loads KS / 4
+    const auto dma_x = [&](int m, half_t* dst) __attribute__((always_inline)) {
+        const int rows = min(16, a.B - 16 * m);
+        const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.lhs) + (int64_t)16 * m * K, 0,
+                                                          (uint32_t)(rows * K * 2), 0x00020000);
+#pragma unroll
+        for (int u = 0; u < KS / 4; ++u) {
+            const int ks = u * 4 + wave;
+            dma_lds<16>(rx, dst + 512 * ks, (uint32_t)((r16 * K + 32 * ks + 8 * g) * 2));
+        }
+    };
+    // the residual and norm of a row block's rows (rows past B, or no residual, read zeros)
+    struct Epi {
+        half8 res;
+        float norm;
+    };
+    const auto fetch_epi = [&](int m, Epi& e) __attribute__((always_inline)) {
+        const int rows = min(16, a.B - 16 * m);
+        const auto rn = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.norm) + (int64_t)16 * m * a.D, 0,
+                                                          (uint32_t)(rows * a.D * 4), 0x00020000);
+        e.norm = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rn, (uint32_t)((r16 * a.D + d) * 4), 0, 0));
+        const half_t* base = a.residual != nullptr ? a.residual + (int64_t)16 * m * N : a.lhs;
+        const auto rr = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(base), 0,
+                                                          a.residual != nullptr ? (uint32_t)(rows * N * 2) : 0u, 0x00020000);
+        e.res = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rr, (uint32_t)((r16 * N + nc) * 2), 0, 0));
+    };
+    Epi e0, e1, e2, e3;
+    const auto block = [&](int m, const half_t* X, half_t* Xn, const Epi& e, Epi& en) __attribute__((always_inline)) {
+        const int mn = min(m + 3, m_end - 1);
+        fetch_epi(mn, en);
+        dma_x(mn, Xn);
+        asm volatile("" ::: "memory");
+        float4v acc[2] = {float4v{bv[0], bv[1], bv[2], bv[3]}, float4v{bv[4], bv[5], bv[6], bv[7]}};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const half8 xb = *reinterpret_cast<const half8*>(X + (ks * kWave + lane) * 8);
+#pragma unroll
+            for (int hb = 0; hb < 2; ++hb) acc[hb] = mfma16x16x32(tw[hb][ks], xb, acc[hb]);
+        }
+        const float inv = 1.f / (a.eps + e.norm);
+        half8 h;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) h[j] = (half_t)(acc[j >> 2][j & 3] * inv + (float)e.res[j]);
+        const int rows = min(16, a.B - 16 * m);
+        const auto ro = __builtin_amdgcn_make_buffer_rsrc(a.out + (int64_t)16 * m * N, 0, (uint32_t)(rows * N * 2), 0x00020000);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, h), ro,
+                                               nin && r16 < rows ? (uint32_t)((r16 * N + n) * 2) : kDrop, 0, 0);
+        // the next block's rows have landed: newer than them are the loads of the two blocks after it
+        // (residual, norm and KS / 4 direct-to-LDS loads each) and three stores
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(3 + 2 * (2 + KS / 4)) : "memory");
+    };
+    if (m_begin >= m_end) return;
+    fetch_epi(m_begin, e0);
+    dma_x(m_begin, X0);
+    fetch_epi(min(m_begin + 1, m_end - 1), e1);
+    dma_x(min(m_begin + 1, m_end - 1), X1);
+    fetch_epi(min(m_begin + 2, m_end - 1), e2);
+    dma_x(min(m_begin + 2, m_end - 1), T0);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * (2 + KS / 4)) : "memory");
+    for (int m = m_begin; m < m_end; m += 4) {
+        block(m, X0, T1, e0, e3);
+        if (m + 1 >= m_end) break;
+        block(m + 1, X1, X0, e1, e0);
+        if (m + 2 >= m_end) break;
+        block(m + 2, T0, X1, e2, e1);
+        if (m + 3 >= m_end) break;
+        block(m + 3, T1, T0, e3, e2);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // ---- opm_outer ----------------------------------------------------------------------------
@@ -312,7 +467,17 @@ extern "C" int clk_opm_update(clk_stream stream, const clk_buffer* lhs, const cl
     if (items > INT32_MAX) return invalid("opm_update: too large");
     const dim3 grid((unsigned)items);
     stage_mark(s, 0);
-    if (K % 128 == 0) {
+    // t^T in registers (opm_update_cols_kernel) pays where each workgroup walks at least eight row
+    // blocks: its rows are split over as many workgroups as fill the 512 places, two on each CU
+    const int64_t ntiles = (D * F + 127) / 128, mblocks = (B + 15) / 16;
+    const int64_t splits = ntiles >= 448 ? 1 : (512 + ntiles - 1) / ntiles, per = (mblocks + splits - 1) / splits;
+    if ((K == 128 || K == 256 || K == 512) && per >= 8 && ntiles * splits <= INT32_MAX) {
+        const dim3 cgrid((unsigned)(ntiles * splits));
+#define CLK_OPM_COLS(KS_)                                                                              \
+        if (K == 32 * KS_) hipLaunchKernelGGL(opm_update_cols_kernel<KS_>, cgrid, dim3(256), 0, s, a, (int)splits, (int)per);
+        CLK_OPM_COLS(4) CLK_OPM_COLS(8) CLK_OPM_COLS(16)
+#undef CLK_OPM_COLS
+    } else if (K % 128 == 0) {
         hipLaunchKernelGGL(opm_update_kernel<128>, grid, dim3(256), 0, s, a);
     } else if (K % 64 == 0) {
         hipLaunchKernelGGL(opm_update_kernel<64>, grid, dim3(256), 0, s, a);

@@ -1,0 +1,40 @@
+"""opm_update where K is 128, 256 or 512 against the float64 oracle: past about 57000 columns, or with
+rows enough to split, t^T is in registers and the lhs rows are streamed. Row blocks and column tiles cut
+short, rows split over workgroups or not, the residual absent, apart and in place.
+"""
+import numpy as np
+import pytest
+import torch
+
+from conftest import abs_excess
+from oracle import opm as oro
+
+pytestmark = pytest.mark.gpu
+
+ATOL = 2e-3  # beyond each fp16 result's half-ulp rounding
+
+
+@pytest.mark.parametrize("k", [128, 256, 512])
+@pytest.mark.parametrize("b,d,f", [(17, 9, 16), (113, 449, 128), (121, 3590, 16), (520, 260, 64)])
+@pytest.mark.parametrize("residual", ["none", "apart", "in place"])
+def test_columns(hip, k, b, d, f, residual):
+    rng = np.random.default_rng(k + b + d + f)
+    lhs = rng.standard_normal((b, k)).astype(np.float16)
+    t = (rng.standard_normal((k, d, f)) * k ** -0.5).astype(np.float16)
+    bias = (rng.standard_normal(f) * 0.1).astype(np.float32)
+    norm = rng.integers(1, k // 32 + 1, size=(b, d)).astype(np.float32)
+    res = None if residual == "none" else (rng.standard_normal((b, d, f)) * 2).astype(np.float16)
+    dev = [torch.from_numpy(a).cuda() for a in (lhs, t, bias, norm)]
+    n = b * d * f
+    store = torch.full((n + 64,), 7.0, dtype=torch.float16, device="cuda")
+    out = store[:n].view(b, d, f)
+    tr = None
+    if res is not None:
+        tr = torch.from_numpy(res).cuda()
+        if residual == "in place":
+            out.copy_(tr)
+            tr = out
+    hip.opm_update(*dev, tr, eps=1e-3, out=out)
+    torch.cuda.synchronize()
+    assert abs_excess(out.float().cpu().numpy(), oro.opm_update(lhs, t, bias, norm, 1e-3, res)) <= ATOL
+    assert (store[n:] == 7.0).all()
