@@ -1176,7 +1176,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
 // at three per SIMD, key group w % 4 by query third w / 4 (four tiles each, two per step), so the
 // dBias partial is 32 registers per lane and the kernel fits 168 VGPRs; for QT = 8 (128 < Sq <=
 // 256) sixteen waves at four per SIMD, key group w % 4 by query quarter w / 4 (two tiles each, one
-// per step), 16 registers of partial within 128 VGPRs. Its LDS holds the workgroup's bias as
+// per step, two at D <= 16), 16 registers of partial within 128 VGPRs. Its LDS holds the workgroup's bias as
 // fp16 (the original values, recovered exactly from the fp32 log2e form), so s2 = log2e (scale S
 // + bias) takes an fma with the fp16 operand read in place and a multiply. The parts' dK / dV
 // sums meet in LDS once per row, parts 1, 2 (, 3) into part 0 in that order.
@@ -1190,6 +1190,8 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
 // run-time D), 16 for D <= 16, else 24. Up to 16, dV^T and dK^T are one block of 16 d's instead of two:
 // half the transposed reads, a quarter of the products and half the row-end sums. Forward + backward
 // at [1024, 8, 256, 8] 610 -> 574 us, [512, 8, 500, 8] 1169 -> 1097, [512, 4, 384, 16] 349 -> 336.
+// The LDS that this frees lets QT = 8 take both tiles of a part in one step, one barrier a row instead of
+// two and the two tiles' chains side by side: [1024, 8, 256, 8] 576 -> 549, [512, 8, 500, 8] 1097 -> 1060.
 //
 // Sq > 384 runs it in query windows (WIN), one launch after another, each QT tiles from wt0 on: a
 // window's dK / dV sums of a row start from the fp32 running sum that the window before left in the
@@ -1199,20 +1201,28 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_reg_kernel(BwdArgs a) {
 // tiles take 871 us (rocprofv3); the LDS-partial kernel in two windows of 10, with a pass that adds up
 // their sums, took 992 + 207.
 // ------------------------------------------------------------------------------------------
-template <int QT>
+template <int QT, int DT>
 struct PartTile {
     static constexpr int kParts = QT == 12 ? 3 : 4;      // query parts (waves per key group)
     static constexpr int kThreads = 4 * kParts * kWave;
-    static constexpr int kTPS = QT == 12 ? 2 : 1;        // tiles per part and step
+    // tiles per part and step: two where LDS allows (QT 8 at D <= 16, whose row-end sums are half the
+    // size: a row is then one step, and they and the buffers alternate by row)
+    static constexpr int kTPS = QT == 12 || DT == 16 ? 2 : 1;
 };
 
 template <int QT, bool DBIAS, bool WIN, int DT>
-__global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn_bwd_dkdv_reg3_kernel(BwdArgs a) {
-    static_assert(QT == 12 || QT == 8, "query parts of two tiles per step (QT 12) or one (QT 8)");
-    constexpr int kParts = PartTile<QT>::kParts, kTPS = PartTile<QT>::kTPS, kNT = PartTile<QT>::kThreads;
+// (aligned: the same code starting 512 bytes past a KB took 1% longer at [512, 8, 384, 32] than on one)
+__attribute__((aligned(1024))) __global__ __launch_bounds__((PartTile<QT, DT>::kThreads), QT == 12 ? 3 : 4) void attn_bwd_dkdv_reg3_kernel(BwdArgs a) {
+    static_assert(QT == 12 || QT == 8, "three or four query parts");
+    using PT = PartTile<QT, DT>;
+    constexpr int kParts = PT::kParts, kTPS = PT::kTPS, kNT = PT::kThreads;
     constexpr int TT = QT / kParts;  // tiles per part
     constexpr int kSteps = TT / kTPS;
-    static_assert(kSteps == 2, "buffer parity alternates by step within a row");
+    static_assert(kSteps == 2 || kSteps == 1, "buffer parity alternates by step, within a row or by row");
+    constexpr int kSlots = kSteps == 1 ? 2 : 1;  // row-end sums, by row parity
+    // d blocks of dV^T and dK^T and the d's of a lane (8 in two blocks, 4 in one): A row r of block db is
+    // d = 8 (r / 4) + 4 db + r % 4, with one block d = r
+    constexpr int kDB = DT == 16 ? 1 : 2, kLD = 4 * kDB;
     constexpr int kTile = 32 * 32, kOs = kTile + 64, kSub = kOs + kTile;
     constexpr int kBuf = kParts * kTPS * kSub;  // halfs of a step: [part][tile]
     constexpr int kQTerms = kParts * kTPS * 16; // float4 slots of a step's query terms
@@ -1221,12 +1231,15 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
     __shared__ __attribute__((aligned(16))) half_t bias_l[65 * kBRow];  // rows: 64 keys, masked
     __shared__ __attribute__((aligned(16))) half_t lds0[kBuf];
     __shared__ __attribute__((aligned(16))) half_t lds1[kBuf];
-    // query terms of each buffer [part][tile][-lse2 / c1 x 32, -delta x 32] (at most 384 of the
-    // first 512 floats), then 384 zeros, the -delta a dead key's lane reads
-    __shared__ __attribute__((aligned(16))) float qterms0[512 + 384];
-    __shared__ __attribute__((aligned(16))) float qterms1[512 + 384];
-    // parts 1 .. kParts - 1's dK / dV sums of a row: [part - 1][key group][float4 j][lane]
-    __shared__ __attribute__((aligned(16))) float4 red[(kParts - 1) * 4 * 2 * (DT == 16 ? 1 : 2) * 64];
+    // query terms of each buffer [part][tile][-lse2 / c1 x 32, -delta x 32] (at most the
+    // first 512 floats), then as many zeros, the -delta a dead key's lane reads
+    constexpr int kZero = kParts * kTPS * 64;
+    static_assert(kZero <= 512 && kZero / 2 <= kNT, "one float4 of zeros a thread");
+    __shared__ __attribute__((aligned(16))) float qterms0[512 + kZero];
+    __shared__ __attribute__((aligned(16))) float qterms1[512 + kZero];
+    // parts 1 .. kParts - 1's dK / dV sums of a row: [slot][part - 1][key group][float4 j][lane]
+    constexpr int kRed = (kParts - 1) * 4 * 2 * kDB * 64;
+    __shared__ __attribute__((aligned(16))) float4 red[kSlots * kRed];
 
     const int item = xcd_item(blockIdx.x, gridDim.x);
     const int rest = fdiv(item, a.fkb), kblk = item - rest * a.kblocks;
@@ -1242,13 +1255,10 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
     const bool kin = key < a.Sk;
     const float c1s = a.c1s;
     const int D = DT == 32 ? 32 : a.D;
-    // d blocks of dV^T and dK^T and the d's of a lane (8 in two blocks, 4 in one): A row r of block db is
-    // d = 8 (r / 4) + 4 db + r % 4, with one block d = r
-    constexpr int kDB = DT == 16 ? 1 : 2, kLD = 4 * kDB;
     const int wt0 = WIN ? a.wt0 : 0;  // the window's first tile
     const int SqR = WIN ? a.SqB : SqB;  // transposed-bias row length
 
-    if (tid < 192) reinterpret_cast<float4*>(tid < 96 ? qterms0 + 512 : qterms1 + 128)[tid] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (tid < kZero / 2) reinterpret_cast<float4*>(tid < kZero / 4 ? qterms0 + 512 : qterms1 + 512 - kZero)[tid] = make_float4(0.f, 0.f, 0.f, 0.f);
 
     // this wave's staging share of a step: tile (part sq3, tile si) of tensor (Q, dO); waves past
     // the step's kParts kTPS tiles x 2 tensors stage none
@@ -1340,9 +1350,14 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
             }
         }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first step's tiles, as at the end of a step
     __syncthreads();
 
-    for (int pass = 0; pass < rows; ++pass) {
+    // kSlots rows an iteration, the first step of row `pass` in buffer `slot`
+    for (int pass = 0; pass < rows; ++pass)
+#pragma unroll
+    for (int slot = 0; slot < kSlots; ++slot) {
+        if (slot > 0 && ++pass >= rows) break;
         const int n = n_begin + pass;
         const bool alive = kin && mbn != 0u;
         const half8 kop = alive && a.kscale ? kopn : bzero8();
@@ -1362,7 +1377,7 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
 
 #pragma unroll
         for (int st = 0; st < kSteps; ++st) {
-            const int par = st & 1;  // kSteps is even
+            const int par = (slot + st) & 1;
             if constexpr (WIN) {
                 if (st == kSteps - 1) {
                     const int64_t plane = (int64_t)a.N * a.H * a.Sk * D, nh = (int64_t)n * a.H + h;
@@ -1443,7 +1458,7 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
                 dvdk(0);
             }
             if (st == kSteps - 1 && q3 > 0) {
-                float4* r = red + ((q3 - 1) * 4 + kg) * 2 * kDB * 64 + lane;
+                float4* r = red + slot * kRed + ((q3 - 1) * 4 + kg) * 2 * kDB * 64 + lane;
 #pragma unroll
                 for (int db = 0; db < kDB; ++db) {
                     r[64 * db] = make_float4(acck[db][0], acck[db][1], acck[db][2], acck[db][3]);
@@ -1461,7 +1476,7 @@ __global__ __launch_bounds__(PartTile<QT>::kThreads, QT == 12 ? 3 : 4) void attn
             // part 0 + part 1 + ... (+ the windows before)
 #pragma unroll
             for (int t = 0; t < kParts - 1; ++t) {
-                const float4* r = red + (t * 4 + kg) * 2 * kDB * 64 + lane;
+                const float4* r = red + slot * kRed + (t * 4 + kg) * 2 * kDB * 64 + lane;
 #pragma unroll
                 for (int db = 0; db < kDB; ++db) {
                     const float4 k0 = r[64 * db], v0 = r[64 * (kDB + db)];
@@ -1853,7 +1868,7 @@ static void launch_dkdv(hipStream_t stream, const BwdArgs& a, const BwdPlan& p, 
 
 template <int QT, bool WIN, int DT>
 static void launch_parts(hipStream_t stream, dim3 grid, const BwdArgs& a, bool want_dbias) {
-    const dim3 threads(PartTile<QT>::kThreads);
+    const dim3 threads(PartTile<QT, DT>::kThreads);
     if (want_dbias) {
         hipLaunchKernelGGL((attn_bwd_dkdv_reg3_kernel<QT, true, WIN, DT>), grid, threads, 0, stream, a);
     } else {

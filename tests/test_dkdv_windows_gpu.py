@@ -18,7 +18,8 @@ GRAD_ATOL = 5e-3  # beyond each fp16 result's half-ulp rounding, as for every ba
 @pytest.mark.parametrize("n,h,sq,sk,d,windows", [
     (3, 2, 100, 90, 8, 1), (2, 2, 128, 65, 16, 1), (2, 3, 140, 60, 16, 1), (2, 2, 257, 64, 24, 1), (700, 1, 384, 33, 8, 1),
     (2, 2, 385, 100, 32, 2), (600, 1, 416, 40, 32, 2), (2, 2, 513, 130, 16, 2), (2, 1, 640, 129, 8, 2), (2, 2, 768, 70, 24, 2),
-    (2, 1, 769, 64, 32, 3), (300, 2, 900, 20, 32, 3)])
+    (2, 1, 769, 64, 32, 3), (300, 2, 900, 20, 32, 3),
+    (700, 1, 200, 33, 8, 1), (1500, 1, 256, 20, 16, 1), (901, 1, 560, 40, 16, 2)])
 def test_register_windows(hip, n, h, sq, sk, d, windows):
     assert hip.attention_bwd_plan(n, h, sq, sk, d)["windows"] == windows
     rng = np.random.default_rng(sq + sk + d)
