@@ -259,7 +259,9 @@ __global__ __launch_bounds__(256, 2) void opm_update_cols_kernel(OpmUpdateArgs a
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, h), ro,
                                                nin && r16 < rows ? (uint32_t)((r16 * N + n) * 2) : kDrop, 0, 0);
         // the next block's rows have landed: newer than them are the loads of the two blocks after it
-        // (residual, norm and KS / 4 direct-to-LDS loads each) and three stores
+        // (residual, norm and KS / 4 direct-to-LDS loads each) and three stores; after the first and
+        // second block only one and two stores
+        if (m < m_begin + 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(1 + 2 * (2 + KS / 4)) : "memory");
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(3 + 2 * (2 + KS / 4)) : "memory");
     };
     if (m_begin >= m_end) return;
