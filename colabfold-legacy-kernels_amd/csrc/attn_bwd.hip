@@ -59,7 +59,7 @@ struct BwdArgs {
     float* dkv;
     int N, H, Sq, Sk, D;
     int SqA, SkA;    // Sq rounded up to 32, Sk rounded up to 64
-    int SqB;         // queries per transposed-bias row: SqA, or 32 QT for the register kernel
+    int SqB;         // queries per transposed-bias row: SqA, or the register kernels' whole windows
     int kblocks;     // ceil(Sk / 64)
     int chunk;       // batch rows per dkdv workgroup
     int chunks;
@@ -1681,6 +1681,7 @@ struct BwdPlan {
     int QT = 0;  // query tiles of the register-partial dK/dV kernel (4, 8 or 12), 0: not used
     int n12 = 0, n8 = 0;  // the register kernel's query windows: n12 of 12 tiles, then n8 of 8
     int QG = 1;  // query groups of the dK/dV kernel
+    int per_cu = 1;  // dK/dV workgroups on a CU
     int kblocks = 0, chunk = 0, chunks = 0;
     int wtiles = 1, windows = 1;  // query windows of the dK/dV kernel
     size_t stage_lds = 0, dbias_lds = 0;
@@ -1752,8 +1753,8 @@ static BwdPlan plan_lds(int device, int64_t N, int64_t H, int64_t Sq, int64_t Sk
     // batch-row chunks: the fewest rounds of workgroups times rows per workgroup
     const size_t per_wg = p.stage_lds + p.dbias_lds;
     const int threads = 256 * p.QG;
-    int per_cu = std::max(1, std::min(2048 / threads, (int)(limit / per_wg)));
-    const int64_t slots = (int64_t)cu_count(device) * per_cu;
+    p.per_cu = std::max(1, std::min(2048 / threads, (int)(limit / per_wg)));
+    const int64_t slots = (int64_t)cu_count(device) * p.per_cu;
     const int64_t cols = std::max<int64_t>(H * p.kblocks * p.windows, 1);
     int64_t best = 1, best_cost = INT64_MAX;
     for (int64_t ch = 1; ch <= Nr; ch = next_chunks(Nr, ch)) {
@@ -1837,17 +1838,45 @@ constexpr size_t kNoAllocScratchBytes = size_t(96) << 20;
 
 static bool reg_only(int64_t Sq, int64_t D) { return D == 32 && Sq <= 384; }
 
+// Whether the LDS-partial kernel can take less time than the register kernels at D <= 32, and whether
+// its plan l is estimated to take less than theirs, r. The register
+// kernels pad the queries to whole windows; past 384 queries they run one launch a window, and each
+// window reads and writes the running sums of dK and dV. At 13 to 15 tiles, where they pad to two
+// windows of 8 and the LDS-partial kernel still has one window, that costs more than it gains at
+// D = 24 and 32 (whole backward at D = 32, LDS-partial and register: [512, 8, 416, 32] 877 and 1019
+// us, [64, 4, 448, 32] 72 and 82), unless the LDS-partial plan has many more dBias partials
+// ([256, 4, 416, 32], 64 chunks against 9: 282 and 257). Both are counted in tile steps of the
+// LDS-partial kernel (about 1 us: each of its row groups takes one tile of a row); a register row of
+// two 8-tile windows is 4.5 of them, a MB of partials written and summed 0.4. Over 160 shapes drawn
+// from 385..480 queries this picks the faster kernel but for 0.2% of the time.
+// Elsewhere the register kernels measured faster ([640, 4, 640, 32]: 871 against 992 + 207 us for
+// dK/dV; [1024, 8, 256, 8]: 319 against 358; D <= 16 at 13 to 15 tiles: 0.65 to 0.99 of the time).
+static bool lds_contends(int64_t Sq, int64_t D) {
+    const int64_t qtiles = (Sq + 31) / 32;
+    return D >= 24 && qtiles >= 13 && qtiles <= 15;
+}
+
+static bool lds_faster(int device, int64_t H, const BwdPlan& l, const BwdPlan& r) {
+    const int64_t cus = cu_count(device), cols = H * r.kblocks;
+    const auto rounds = [&](int64_t chunks, int64_t slots) { return (chunks * cols + slots - 1) / slots; };
+    const auto partials = [&](const BwdPlan& p) { return 0.4e-6 * (double)p.partial_bytes; };
+    const int64_t passes = (l.chunk + l.QG - 1) / l.QG;
+    const double tl = (double)(rounds(l.chunks, cus * l.per_cu) * l.per_cu * passes * l.wtiles) + partials(l);
+    const double tr = 4.5 * (double)(rounds(r.chunks, cus) * r.chunk) + partials(r);
+    return tl <= tr;
+}
+
 // The dK/dV kernel's shape depends only on the problem and the device, never on want_dbias or the
-// entry point, so dk and dv are bit-identical with and without dbias, and with either scratch.
-// D <= 32 takes the register kernels, which measured faster than the LDS-partial one at every size
-// ([640, 4, 640, 32]: 871 against 992 + 207 us; [1024, 8, 256, 8]: 319 against 358), unless
-// only the latter's scratch fits clk_attention_bwd_noalloc's.
+// entry point, so dk and dv are bit-identical with and without dbias, and with either scratch: a
+// shape that clk_attention_bwd_noalloc takes runs a plan that fits its scratch from both entry points.
 static BwdPlan plan_bwd(int device, int64_t N, int64_t H, int64_t Sq, int64_t Sk, int64_t D) {
     if (D > 32) return plan_lds(device, N, H, Sq, Sk, D);
     const BwdPlan r = plan_reg(device, N, H, Sq, Sk, D);
-    if (reg_only(Sq, D) || bwd_workspace_bytes(r) <= kNoAllocScratchBytes) return r;
+    const bool fits = bwd_workspace_bytes(r) <= kNoAllocScratchBytes, contends = lds_contends(Sq, D);
+    if (reg_only(Sq, D) || (fits && !contends)) return r;
     const BwdPlan l = plan_lds(device, N, H, Sq, Sk, D);
-    return bwd_workspace_bytes(l) <= kNoAllocScratchBytes ? l : r;
+    if (contends && lds_faster(device, H, l, r)) return l;
+    return !fits && bwd_workspace_bytes(l) <= kNoAllocScratchBytes ? l : r;
 }
 
 template <int DP, int QG>
@@ -1978,7 +2007,7 @@ extern "C" int clk_attention_bwd_plan(int32_t device, int64_t N, int64_t H, int6
     if (plan == nullptr || count < 0) return invalid("attention_bwd_plan: no output array");
     const BwdPlan p = plan_bwd(device, N, H, Sq, Sk, D);
     const int64_t vals[] = {p.QG, p.chunk, p.chunks, (p.chunk + p.QG - 1) / p.QG, p.windows,
-                            p.QT > 0 && p.windows == 1 ? 1 : 0};
+                            p.QT > 0 ? 1 : 0};
     for (int i = 0; i < count && i < 6; ++i) plan[i] = vals[i];
     return ok();
 }
@@ -2057,9 +2086,10 @@ static int attention_bwd_impl(clk_stream stream, int32_t device, const clk_buffe
     if (N * H * Sq == 0 && N * H * Sk == 0 && H * Sq * Sk == 0) return ok();  // nothing to write
     const size_t need = bwd_workspace_bytes(p);
     if (noalloc) {
-        // (the register windows need less than the LDS-partial kernel's; the shapes that this entry
-        // point takes are still those whose LDS-partial scratch fits)
-        const size_t ask = reg_only(Sq, D) ? need : std::max(need, bwd_workspace_bytes(plan_lds(device, N, H, Sq, Sk, D)));
+        // (which shapes this entry point takes is decided by the LDS-partial kernel's scratch but at
+        // D = 32 and Sq <= 384, whichever kernel runs: a shape's answer does not move with plan_bwd's
+        // choice)
+        const size_t ask = D > 32 || reg_only(Sq, D) ? need : std::max(need, bwd_workspace_bytes(plan_lds(device, N, H, Sq, Sk, D)));
         if (ask > kNoAllocScratchBytes) {
             return invalid("attention_bwd_noalloc: these shapes need " + std::to_string(ask) +
                            " bytes of scratch, the library's static scratch holds " +

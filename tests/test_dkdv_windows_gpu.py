@@ -1,7 +1,8 @@
-"""The register dK/dV kernels at head dims below 32 and in query windows (Sq > 384), against the
-float64 oracle: window edges and ragged last tiles, several rows per workgroup, and the running sum
-of dK and dV that a window hands to the next. dk and dv must not depend on want_dbias, repeat bit for
-bit, and be the same from clk_attention_bwd_noalloc.
+"""The dK/dV kernels at head dims up to 32 where the route is chosen by estimated time, against the
+float64 oracle: the register kernels at head dims below 32 and in query windows (Sq > 384), with window
+edges and ragged last tiles, several rows per workgroup, and the running sum of dK and dV that a window
+hands to the next; and the LDS-partial kernel, over several passes of its row groups. dk and dv must
+not depend on want_dbias, repeat bit for bit, and be the same from clk_attention_bwd_noalloc.
 """
 import numpy as np
 import pytest
@@ -17,11 +18,28 @@ GRAD_ATOL = 5e-3  # beyond each fp16 result's half-ulp rounding, as for every ba
 
 @pytest.mark.parametrize("n,h,sq,sk,d,windows", [
     (3, 2, 100, 90, 8, 1), (2, 2, 128, 65, 16, 1), (2, 3, 140, 60, 16, 1), (2, 2, 257, 64, 24, 1), (700, 1, 384, 33, 8, 1),
-    (2, 2, 385, 100, 32, 2), (600, 1, 416, 40, 32, 2), (2, 2, 513, 130, 16, 2), (2, 1, 640, 129, 8, 2), (2, 2, 768, 70, 24, 2),
+    (2, 2, 385, 100, 32, 2), (600, 1, 520, 40, 32, 2), (2, 2, 513, 130, 16, 2), (2, 1, 640, 129, 8, 2), (2, 2, 768, 70, 24, 2),
     (2, 1, 769, 64, 32, 3), (300, 2, 900, 20, 32, 3),
     (700, 1, 200, 33, 8, 1), (1500, 1, 256, 20, 16, 1), (901, 1, 560, 40, 16, 2)])
 def test_register_windows(hip, n, h, sq, sk, d, windows):
-    assert hip.attention_bwd_plan(n, h, sq, sk, d)["windows"] == windows
+    plan = hip.attention_bwd_plan(n, h, sq, sk, d)
+    assert plan["registers"] == 1 and plan["windows"] == windows, plan
+    compare(hip, n, h, sq, sk, d)
+
+
+@pytest.mark.parametrize("n,h,sq,sk,d,registers,passes", [
+    # 13 to 15 query tiles at D >= 24: the LDS-partial kernel (one row of a pass absent, ragged Sq)
+    (64, 4, 400, 400, 32, 0, 2), (600, 1, 416, 40, 32, 0, 1), (61, 4, 390, 400, 24, 0, 2), (99, 2, 480, 470, 32, 0, 2),
+    # but where its plan has the many more partials, few rows, or 16 tiles or 12
+    (256, 4, 386, 400, 32, 1, 29), (2, 2, 385, 100, 32, 1, 1), (64, 4, 481, 470, 32, 1, 8), (64, 4, 384, 400, 32, 1, 8)])
+def test_route(hip, n, h, sq, sk, d, registers, passes):
+    plan = hip.attention_bwd_plan(n, h, sq, sk, d)
+    assert plan["registers"] == registers and plan["passes"] == passes, plan
+    if n * h * sq * sk <= 6e7:  # the oracle's time
+        compare(hip, n, h, sq, sk, d)
+
+
+def compare(hip, n, h, sq, sk, d):
     rng = np.random.default_rng(sq + sk + d)
     f16 = lambda *shape: (rng.standard_normal(shape) * 0.5).astype(np.float16)
     q, k, v, bias, dout = f16(n, h, sq, d), f16(n, h, sk, d), f16(n, h, sk, d), f16(h, sq, sk), f16(n, h, sq, d)
