@@ -1849,20 +1849,27 @@ static bool reg_only(int64_t Sq, int64_t D) { return D == 32 && Sq <= 384; }
 // LDS-partial kernel (about 1 us: each of its row groups takes one tile of a row); a register row of
 // two 8-tile windows is 4.5 of them, a MB of partials written and summed 0.4. Over 160 shapes drawn
 // from 385..480 queries this picks the faster kernel but for 0.2% of the time.
+// At D < 32 and one or two tiles the LDS-partial kernel runs, with as many row groups as tiles: the
+// register kernel pads to four ([191, 1, 47, 24] 25 us against 19, [409, 8, 35 x 282, 8] 123 against
+// 91; over 122 drawn shapes 2% slower). At D = 24 and 5 or 6 tiles, padded to 8, the plans are compared
+// too ([512, 8, 192, 24] 192 us against 183, but [144, 8, 158 x 99, 24] 47 against 64); a register row
+// of one 8-tile window is 1.7 steps.
 // Elsewhere the register kernels measured faster ([640, 4, 640, 32]: 871 against 992 + 207 us for
 // dK/dV; [1024, 8, 256, 8]: 319 against 358; D <= 16 at 13 to 15 tiles: 0.65 to 0.99 of the time).
 static bool lds_contends(int64_t Sq, int64_t D) {
     const int64_t qtiles = (Sq + 31) / 32;
-    return D >= 24 && qtiles >= 13 && qtiles <= 15;
+    return (D >= 24 && qtiles >= 13 && qtiles <= 15) || (D < 32 && qtiles <= 2) ||
+           (D == 24 && (qtiles == 5 || qtiles == 6));
 }
 
 static bool lds_faster(int device, int64_t H, const BwdPlan& l, const BwdPlan& r) {
+    if (r.wtiles <= 2) return true;
     const int64_t cus = cu_count(device), cols = H * r.kblocks;
     const auto rounds = [&](int64_t chunks, int64_t slots) { return (chunks * cols + slots - 1) / slots; };
     const auto partials = [&](const BwdPlan& p) { return 0.4e-6 * (double)p.partial_bytes; };
     const int64_t passes = (l.chunk + l.QG - 1) / l.QG;
     const double tl = (double)(rounds(l.chunks, cus * l.per_cu) * l.per_cu * passes * l.wtiles) + partials(l);
-    const double tr = 4.5 * (double)(rounds(r.chunks, cus) * r.chunk) + partials(r);
+    const double tr = (r.windows > 1 ? 4.5 : 1.7) * (double)(rounds(r.chunks, cus) * r.chunk) + partials(r);
     return tl <= tr;
 }
 

@@ -31,7 +31,11 @@ def test_register_windows(hip, n, h, sq, sk, d, windows):
     # 13 to 15 query tiles at D >= 24: the LDS-partial kernel (one row of a pass absent, ragged Sq)
     (64, 4, 400, 400, 32, 0, 2), (600, 1, 416, 40, 32, 0, 1), (61, 4, 390, 400, 24, 0, 2), (99, 2, 480, 470, 32, 0, 2),
     # but where its plan has the many more partials, few rows, or 16 tiles or 12
-    (256, 4, 386, 400, 32, 1, 29), (2, 2, 385, 100, 32, 1, 1), (64, 4, 481, 470, 32, 1, 8), (64, 4, 384, 400, 32, 1, 8)])
+    (256, 4, 386, 400, 32, 1, 29), (2, 2, 385, 100, 32, 1, 1), (64, 4, 481, 470, 32, 1, 8), (64, 4, 384, 400, 32, 1, 8),
+    # one or two tiles at D < 32: the LDS-partial kernel with one or two row groups; three not
+    (3000, 1, 31, 33, 8, 0, 11), (1111, 2, 64, 64, 16, 0, 3), (751, 1, 33, 130, 24, 0, 3), (300, 1, 65, 64, 24, 1, 2),
+    # 5 and 6 tiles at D = 24
+    (561, 8, 164, 136, 24, 0, 7), (850, 4, 142, 142, 24, 0, 6), (144, 8, 158, 99, 24, 1, 9), (150, 4, 190, 200, 16, 1, 10)])
 def test_route(hip, n, h, sq, sk, d, registers, passes):
     plan = hip.attention_bwd_plan(n, h, sq, sk, d)
     assert plan["registers"] == registers and plan["passes"] == passes, plan
