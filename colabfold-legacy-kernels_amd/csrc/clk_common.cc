@@ -61,6 +61,20 @@ int shared_limit(int device) {
     return g_shared_limit[device];
 }
 
+int current_cu_count() {
+    static int cus = 0;
+    if (cus == 0) {
+        int dev = 0, v = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) {
+            cus = v;
+        } else {
+            cus = 256;
+        }
+    }
+    return cus;
+}
+
 int check_types(const char* what, const clk_buffer* const* bufs, const int* types, int n) {
     for (int i = 0; i < n; ++i) {
         if (bufs[i] == nullptr) {

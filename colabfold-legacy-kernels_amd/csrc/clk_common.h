@@ -216,6 +216,9 @@ void stage_mark(hipStream_t s, int i);
 // per-device caches).
 int shared_limit(int device);
 
+// The current device's CUs (those of the first call; 256 where they cannot be read).
+int current_cu_count();
+
 inline int64_t elements(const clk_buffer* b) {
     int64_t n = 1;
     for (int i = 0; i < b->rank; ++i) n *= b->dims[i];

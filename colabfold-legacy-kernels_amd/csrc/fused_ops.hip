@@ -1811,20 +1811,6 @@ __global__ __launch_bounds__(kTransRowsThreads, 4) void transition_rows_kernel(T
 
 // ---- host side --------------------------------------------------------------------------------
 
-static int fused_cu_count() {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) {
-            cus = v;
-        } else {
-            cus = 256;
-        }
-    }
-    return cus;
-}
-
 static int fused_lds_limit() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
@@ -1856,7 +1842,7 @@ static unsigned persistent_grid(int64_t tiles, size_t lds, int max_per_cu = 4) {
     const int limit = fused_lds_limit();
     int per_cu = std::min(2, max_per_cu);
     if (limit > 0 && lds > 0) per_cu = std::max(1, std::min(max_per_cu, (int)(limit / lds)));
-    const int64_t g = std::min<int64_t>(tiles, (int64_t)fused_cu_count() * per_cu);
+    const int64_t g = std::min<int64_t>(tiles, (int64_t)current_cu_count() * per_cu);
     return (unsigned)std::max<int64_t>(g, 1);
 }
 
@@ -2189,7 +2175,7 @@ static int run_transition_rows(const TransArgs& a, hipStream_t s) {
 template <int C, int RB, int WV, bool ADD, bool BF>
 static int run_transition_stream(const TransArgs& a, hipStream_t s) {
     const int64_t tiles = ((int64_t)a.M + WV * RB * 16 - 1) / (WV * RB * 16);
-    const dim3 grid((unsigned)std::min<int64_t>(tiles, fused_cu_count()));
+    const dim3 grid((unsigned)std::min<int64_t>(tiles, current_cu_count()));
     stage_mark(s, 0);
     hipLaunchKernelGGL((transition_stream_kernel<C, RB, WV, ADD, BF>), grid, dim3(WV * kWave), 0, s, a);
     stage_mark(s, 1);
@@ -2210,7 +2196,7 @@ static int run_transition(const TransArgs& a, hipStream_t s) {
         // 128-row tiles where one round of them covers M, 256-row tiles past that: a round of 256-row
         // tiles takes 59 us at C = 256, H = 4 C (21 at C = 128), one of 128-row tiles 43 (18), whose
         // fragment reads feed one product each
-        if (a.M <= 128 * fused_cu_count()) return run_transition_stream<C, 1, 8, ADD, BF>(a, s);
+        if (a.M <= 128 * current_cu_count()) return run_transition_stream<C, 1, 8, ADD, BF>(a, s);
         return run_transition_stream<C, 2, 8, ADD, BF>(a, s);
     }
 }

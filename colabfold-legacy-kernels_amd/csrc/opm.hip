@@ -135,12 +135,11 @@ __global__ __launch_bounds__(256) void opm_update_kernel(OpmUpdateArgs a) {
 // buffers, three blocks ahead. So t comes from HBM once and no row block waits for it again, a row
 // block's operand read feeds both of the wave's column blocks, and a row block costs one barrier; the
 // tiled kernel above stages every K step of both operands between two barriers.
-// The rows are split over workgroups that share a column tile (and t through L2) until those fill the
-// places for them.
+// The rows are split over workgroups that share a column tile (and t through L2); cols_plan chooses how many.
 // The residual and norm of a row block are loaded with its lhs rows (loads complete in issue order, so
 // a later load of theirs would be waited for with everything before it).
-// K = 512, F = 128 (us, the tiled kernel's time first): B = D = 509 98.5 -> 71.6, 384 62 -> 53, 256 25.2 ->
-// 23.8; B = D = 128, where a workgroup would walk two blocks, 10.3 -> 12.9 and stays with the tiled kernel.
+// K = 512, F = 128 (us, the tiled kernel's time first): B = D = 512 80.7 -> 62.3, 384 47.3 -> 40.4, 256 24.5 ->
+// 21.8; with few row blocks forming t^T does not pay.
 template <int KS>
 __global__ __launch_bounds__(256, 2) void opm_update_cols_kernel(OpmUpdateArgs a, int splits, int blocks_per) {
     constexpr int K = 32 * KS, kCh = K / 64;  // 64-row chunks of t, 16 KB of a workgroup's columns each
@@ -430,6 +429,37 @@ __global__ __launch_bounds__(256) void opm_outer_kernel(OpmOuterArgs a) {
         }
 }
 
+// Whether opm_update_cols_kernel serves these sizes, and how many workgroups share a column tile's row
+// blocks: the split with the least estimated time, where that is below 0.9 of the tiled kernel's. Both
+// are in us, as measured on 256 CUs, by whole rounds of the CUs. Of the columns kernel two workgroups
+// share a CU, and one alone takes its row blocks twice as fast, so an odd round counts for about half;
+// a workgroup's cost is forming t^T and a step per row block, both linear in K. The tiled kernel's is
+// that of a 64 x 64 tile. A workgroup walks at least 8 row blocks: with fewer the estimate is not to be
+// relied on ([105 x 834, 128] at K = 256, 7 blocks: 23.2 us against 20.7 tiled). Over 260 drawn sizes
+// (60 to 1300 rows, up to 2000 x 128 columns, each K) the rule takes 0.896 of the tiled kernel's
+// time (always the faster of both and the best split: 0.861), and is slower than it by 4 to 7% at 3 of
+// them. Filling 512 places whatever the rounds took 0.944 and was slower by 2 to 17% at 25: 595
+// workgroups, say, run as long as 1024 (K = 512, [899 x 170, 64]: 32 us against 28 by the tiled kernel).
+static bool cols_plan(int64_t B, int64_t K, int64_t D, int64_t F, int64_t tiled_items, int* splits, int* per) {
+    if (K != 128 && K != 256 && K != 512) return false;
+    const int64_t cus = current_cu_count(), ntiles = (D * F + 127) / 128, mblocks = (B + 15) / 16;
+    const auto rounds = [&](int64_t n) { return (n + cus - 1) / cus; };
+    const double k = (double)K;
+    double best = 1e300;
+    for (int64_t sp = 1; sp <= 12; ++sp) {
+        const int64_t p = (mblocks + sp - 1) / sp, r = rounds(ntiles * sp);
+        if (p < 8 || (sp > 1 && r > 4)) break;
+        const double t = 1.5 + (double)(r / 2) * (0.8 + 0.0098 * k + (double)p * (0.49 + 0.0018 * k)) +
+                         (double)(r % 2) * (0.8 + 0.0062 * k + (double)p * (0.24 + 0.00088 * k));
+        if (t < best) {
+            best = t;
+            *splits = (int)sp;
+            *per = (int)p;
+        }
+    }
+    return best < 0.9 * (3.0 + (double)rounds(tiled_items) * (0.64 + 0.00343 * k));
+}
+
 static bool opm_width(int64_t f) { return f == 16 || f == 32 || f == 64 || f == 128; }
 
 }  // namespace clk
@@ -469,14 +499,11 @@ extern "C" int clk_opm_update(clk_stream stream, const clk_buffer* lhs, const cl
     if (items > INT32_MAX) return invalid("opm_update: too large");
     const dim3 grid((unsigned)items);
     stage_mark(s, 0);
-    // t^T in registers (opm_update_cols_kernel) pays where each workgroup walks at least eight row
-    // blocks: its rows are split over as many workgroups as fill the 512 places, two on each CU
-    const int64_t ntiles = (D * F + 127) / 128, mblocks = (B + 15) / 16;
-    const int64_t splits = ntiles >= 448 ? 1 : (512 + ntiles - 1) / ntiles, per = (mblocks + splits - 1) / splits;
-    if ((K == 128 || K == 256 || K == 512) && per >= 8 && ntiles * splits <= INT32_MAX) {
-        const dim3 cgrid((unsigned)(ntiles * splits));
+    int splits = 0, per = 0;
+    if (cols_plan(B, K, D, F, items, &splits, &per)) {
+        const dim3 cgrid((unsigned)((D * F + 127) / 128 * splits));
 #define CLK_OPM_COLS(KS_)                                                                              \
-        if (K == 32 * KS_) hipLaunchKernelGGL(opm_update_cols_kernel<KS_>, cgrid, dim3(256), 0, s, a, (int)splits, (int)per);
+        if (K == 32 * KS_) hipLaunchKernelGGL(opm_update_cols_kernel<KS_>, cgrid, dim3(256), 0, s, a, splits, per);
         CLK_OPM_COLS(4) CLK_OPM_COLS(8) CLK_OPM_COLS(16)
 #undef CLK_OPM_COLS
     } else if (K % 128 == 0) {

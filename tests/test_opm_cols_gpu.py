@@ -1,6 +1,6 @@
-"""opm_update where K is 128, 256 or 512 against the float64 oracle: past about 57000 columns, or with
-rows enough to split, t^T is in registers and the lhs rows are streamed. Row blocks and column tiles cut
-short, rows split over workgroups or not, the residual absent, apart and in place.
+"""opm_update where K is 128, 256 or 512 against the float64 oracle: but for small products t^T is in
+registers and the lhs rows are streamed. Row blocks and column tiles cut short, rows split over
+workgroups or not, the residual absent, apart and in place.
 """
 import numpy as np
 import pytest
@@ -15,7 +15,9 @@ ATOL = 2e-3  # beyond each fp16 result's half-ulp rounding
 
 
 @pytest.mark.parametrize("k", [128, 256, 512])
-@pytest.mark.parametrize("b,d,f", [(17, 9, 16), (113, 449, 128), (121, 3590, 16), (520, 260, 64)])
+@pytest.mark.parametrize("b,d,f", [(17, 9, 16), (113, 449, 128), (121, 3590, 16), (520, 260, 64),
+                                   # too few row blocks, one round of half the places, splits with a last workgroup cut short
+                                   (65, 1500, 32), (161, 161, 128), (1000, 33, 64), (1290, 70, 64), (899, 170, 64)])
 @pytest.mark.parametrize("residual", ["none", "apart", "in place"])
 def test_columns(hip, k, b, d, f, residual):
     rng = np.random.default_rng(k + b + d + f)
