@@ -1364,7 +1364,7 @@ constexpr size_t trans_lds_bytes(int C, int H) {
     return (size_t)2 * 2 * hc * C * 2 + (size_t)(3 * C + H) * 4;
 }
 
-template <int C, int RB, int WV, bool ADD, bool BF>
+template <int C, int RB, int WV, bool ADD, bool BF, bool KEEP>
 __global__ __launch_bounds__(WV * kWave, 2) void transition_stream_kernel(TransArgs a) {
     constexpr int KS = C / 32, NCB = C / 16, HC = trans_chunk<C>(), kRows = RB * 16, NG = RB == 1 ? 4 : 2;
     constexpr int kUnit = C > 128 ? 32 : 64;           // keep granularity
@@ -1383,7 +1383,6 @@ __global__ __launch_bounds__(WV * kWave, 2) void transition_stream_kernel(TransA
     const int r16 = lane & 15, g = lane >> 4;
     const int tiles = (a.M + WV * kRows - 1) / (WV * kRows);
     const int chunks = a.H / HC;  // even: H is 2 C or 4 C
-    const bool has_keep = a.keep != nullptr;
 
     // chunk j into buffer buf: fragment t < kF1 is w1's (hidden block t / KS, step t % KS), then w2's
     // (channel block, step of 32 hidden units); every wave loads (kF1 + kF2) / WV of them
@@ -1418,6 +1417,11 @@ __global__ __launch_bounds__(WV * kWave, 2) void transition_stream_kernel(TransA
     constexpr bool kNext = C == 128;
     half8 xop[RB][KS], xn[kNext ? RB : 1][KS];
     half_t kraw = (half_t)1.f;
+    // with keep values, those of the workgroup's whole tile too (WV kRows / 64 a lane), so that each wave
+    // knows without a barrier, which would wait for the loads in flight, whether any has rows to compute
+    constexpr int kTK = KEEP ? WV * kRows / kWave : 1;
+    half_t ktile[kTK];
+    const auto rkeep = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.keep), 0, (uint32_t)a.M * 2u, 0x00020000);
     const auto fetch_block = [&](int t, int rb, half8 (&x)[KS]) __attribute__((always_inline)) {
         const half_t* px = a.x + (int64_t)min((t * WV + wave) * kRows + 16 * rb + r16, a.M - 1) * C + 8 * g;
 #pragma unroll
@@ -1429,7 +1433,13 @@ __global__ __launch_bounds__(WV * kWave, 2) void transition_stream_kernel(TransA
     };
     const auto fetch_keep = [&](int t) __attribute__((always_inline)) {
         const int u0 = ((t * WV + wave) * kRows) & ~(kUnit - 1);
-        if (has_keep) kraw = a.keep[min(u0 + (lane & (kUnit - 1)), a.M - 1)];
+        if constexpr (KEEP) {
+            kraw = a.keep[min(u0 + (lane & (kUnit - 1)), a.M - 1)];
+#pragma unroll
+            for (int i = 0; i < kTK; ++i)  // (rows past M read zeros)
+                ktile[i] = __builtin_bit_cast(half_t, __builtin_amdgcn_raw_buffer_load_b16(
+                    rkeep, (uint32_t)(t * WV * kRows + i * kWave + lane) * 2u, 0, 0));
+        }
     };
 
     int t = blockIdx.x;
@@ -1450,6 +1460,13 @@ __global__ __launch_bounds__(WV * kWave, 2) void transition_stream_kernel(TransA
         const float kv = (m0 & ~(kUnit - 1)) + (lane & (kUnit - 1)) < a.M ? (float)kraw : -1.f;
         const bool any_live = __any(kv > 0.f), any_zero = __any(kv == 0.f);
         const int work = any_live ? (int)kCompute : any_zero ? (int)kPadding : (int)kSkip;
+        bool any = true;
+        if constexpr (KEEP) {
+            bool live = false;
+#pragma unroll
+            for (int i = 0; i < kTK; ++i) live |= (float)ktile[i] > 0.f;
+            any = __any(live);
+        }
         half8 xr[kNext && ADD ? RB : 1][KS];  // the raw rows
         if constexpr (kNext) {
 #pragma unroll
@@ -1511,7 +1528,6 @@ __global__ __launch_bounds__(WV * kWave, 2) void transition_stream_kernel(TransA
         const int nt = t + gridDim.x, ft = min(nt, tiles - 1);
         if constexpr (kNext) {
             fetch(ft);
-            fetch_keep(ft);
         }
         // the output starts from b2: channel 32 (cb / 2) + 8 g + 4 (cb % 2) + i of row (rb, r16)
         float4v acc[NCB][RB];
@@ -1577,7 +1593,8 @@ __global__ __launch_bounds__(WV * kWave, 2) void transition_stream_kernel(TransA
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
-        for (int j = 0; j < chunks; j += 2) {
+        // (a tile of which no wave has anything to compute streams no weights: chunk 0 stays in Wa)
+        for (int j = 0; any && j < chunks; j += 2) {
             dma(j + 1, Wb);
             if (work == kCompute) chunk(Wa, b1s + HC * j);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1587,10 +1604,8 @@ __global__ __launch_bounds__(WV * kWave, 2) void transition_stream_kernel(TransA
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
         }
-        if constexpr (!kNext) {
-            fetch(ADD ? t : ft);
-            fetch_keep(ft);
-        }
+        if constexpr (!kNext) fetch(ADD ? t : ft);
+        fetch_keep(ft);
         const int rows = max(min(kRows, a.M - m0), 0);
         const auto ro = __builtin_amdgcn_make_buffer_rsrc(a.out + (int64_t)m0 * C, 0, (uint32_t)(rows * C) * 2u, 0x00020000);
         const bool store = work == kCompute || (!ADD && work == kPadding);
@@ -2177,7 +2192,11 @@ static int run_transition_stream(const TransArgs& a, hipStream_t s) {
     const int64_t tiles = ((int64_t)a.M + WV * RB * 16 - 1) / (WV * RB * 16);
     const dim3 grid((unsigned)std::min<int64_t>(tiles, current_cu_count()));
     stage_mark(s, 0);
-    hipLaunchKernelGGL((transition_stream_kernel<C, RB, WV, ADD, BF>), grid, dim3(WV * kWave), 0, s, a);
+    if (a.keep != nullptr) {
+        hipLaunchKernelGGL((transition_stream_kernel<C, RB, WV, ADD, BF, true>), grid, dim3(WV * kWave), 0, s, a);
+    } else {
+        hipLaunchKernelGGL((transition_stream_kernel<C, RB, WV, ADD, BF, false>), grid, dim3(WV * kWave), 0, s, a);
+    }
     stage_mark(s, 1);
     return launch_status("transition");
 }

@@ -69,3 +69,28 @@ def test_keep_units(hip, c, add, m):
 def test_dispatch_line(hip, c, m):
     rows = np.unique(np.concatenate([np.arange(300), np.arange(m - 300, m), np.random.default_rng(0).choice(m, 300)]))
     run(hip, c, 4, m, True, None, True, rows)
+
+
+@pytest.mark.parametrize("c", [128, 256])
+def test_padding_costs_no_products(hip, c):
+    """Whole tiles of padding are only stored: the same call with every row kept takes several times as
+    long (256 rows a tile, each of whose products read all weights)."""
+    m = 131072
+    rng = np.random.default_rng(0)
+    dev = [torch.from_numpy(a).cuda() for a in (
+        rng.standard_normal((m, c)).astype(np.float16), np.ones(c, np.float32), np.zeros(c, np.float32),
+        (rng.standard_normal((4 * c, c)) * c ** -.5).astype(np.float16), np.zeros(4 * c, np.float16),
+        orf.w2_blocked((rng.standard_normal((4 * c, c)) * c ** -.5).astype(np.float16)), np.zeros(c, np.float16))]
+    out, ms = torch.empty_like(dev[0]), {}
+    for value in (1, 0) * 4:
+        keep = torch.full((m,), value, dtype=torch.float16, device="cuda")
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        hip.transition(*dev, keep=keep, eps=EPS, out=out)
+        a.record()
+        for _ in range(20):
+            hip.transition(*dev, keep=keep, eps=EPS, out=out)
+        b.record()
+        b.synchronize()
+        ms[value] = min(ms.get(value, 1e9), a.elapsed_time(b))
+        assert value or not out.any()
+    assert ms[0] < 0.7 * ms[1], ms
