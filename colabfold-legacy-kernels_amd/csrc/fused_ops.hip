@@ -1358,8 +1358,10 @@ struct TransArgs {
 //   go to an offset past the tile's end, which the hardware drops.
 // Reading the fragments a group ahead of their products took 11% off, the rows' own registers another 8%
 // with add_input at C = 128. Against the kernel before (the row tile in LDS, weight chunks through
-// registers between two barriers; at C = 256 one wave per SIMD): C = 256, H = 1024, M = 127508: 331 ->
-// 140 us (0.96 PFLOP/s); C = 128, H = 512, M = 262144, bf16 with add_input: 102 -> 83 us (0.83 PFLOP/s).
+// registers between two barriers; at C = 256 one wave per SIMD): C = 256, H = 1024, M = 127508 with
+// add_input: 327 -> 130 us (1.03 PFLOP/s); C = 128, H = 512, M = 262144, bf16 with add_input: 97 -> 80 us
+// (0.86 PFLOP/s). A tile of padding alone streams no weights, as the kernel before skipped it: C = 128,
+// M = 71917 with the last ninth padded 33 us with the weights streamed, 26 without.
 // At M = 262144 neither the matrix cores (27 us at their nominal rate, 56 at a large library product's)
 // nor LDS reads (27 us) bound it alone: the eight waves meet at a barrier per chunk.
 template <int C>

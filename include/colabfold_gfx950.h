@@ -100,7 +100,8 @@ size_t clk_attention_bwd_workspace_size(int32_t device, const clk_buffer* q, con
  * (96 MiB, enough for [512, 8, 384, 32]), held until the process ends. The array is part of the
  * library's code object, so loading the library reserves those 96 MiB on every GPU it runs a
  * kernel on, whether or not this entry point is ever called. Shapes whose scratch
- * would exceed it are rejected with CLK_INVALID_ARGUMENT before any launch. The call allocates
+ * would exceed it are rejected with CLK_INVALID_ARGUMENT before any launch (but at D = 32 and Sq <=
+ * 384, that of the kernel with its dBias partial in LDS, whichever runs). The call allocates
  * nothing. Every call on a GPU shares that GPU's scratch, so calls that overlap on one GPU (two
  * streams, or two threads) race and must be serialised by the caller. */
 int clk_attention_bwd_noalloc(clk_stream stream, int32_t device, const clk_buffer* q,
