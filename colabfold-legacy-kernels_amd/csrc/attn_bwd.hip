@@ -422,8 +422,8 @@ __global__ __launch_bounds__(DqTile<DP>::kThreads, DP == 32 ? 4 : 1) void attn_b
         __builtin_amdgcn_s_waitcnt(kWaitVm0);
         __syncthreads();
     }
-    // a wave whose queries all lie past Sq only stages its share of the key tiles
-    if (wq >= a.Sq) {
+    // a wave whose queries all lie past Sq only stages its share of the key tiles, where idle_waves says so
+    if (wq >= a.Sq && idle_waves(gridDim.x, a.fqt.d)) {
         for (int k0 = 0, buf = 0; k0 < a.Sk; k0 += T::kBK, buf ^= 1) {
             const uint64_t keep_next = __ballot(mbyte != 0u);
             if (k0 + T::kBK < a.Sk) {

@@ -729,10 +729,9 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
         }
         stage(0, 0, keep_cur);
         __syncthreads();
-        // A wave whose 32 queries all lie past Sq only stages its share of the key tiles, in a loop of
-        // its own, so that the other waves' loop carries no branch for it. 240 -> 232 us at [520, 520, 4,
-        // 4, 32], whose fifth query tile holds 8 queries; 94 -> 89 at 256 rows of 272, 8 heads of 32.
-        if (q0 + wv * (T::kQB * 16) >= a.Sq) {
+        // A wave whose 32 queries all lie past Sq only stages its share of the key tiles, where idle_waves
+        // says so, in a loop of its own, so that the other waves' loop carries no branch for it.
+        if (q0 + wv * (T::kQB * 16) >= a.Sq && idle_waves(gridDim.x, a.fqt.d)) {
             for (int k0 = 0, buf = 0; k0 < k_end; k0 += T::kBK, buf ^= 1) {
                 if (k0 + T::kBK < k_end) {
                     fetch_kv(k0 + T::kBK, buf ^ 1);

@@ -103,6 +103,19 @@ __device__ __forceinline__ half8 lds_operand_tr(At at, int g, int lane16, int co
     return half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
+// Whether an attention kernel's waves that have no query (of a last tile that Sq cuts short) skip the
+// products and only stage keys: where every workgroup is such a one (a single query tile a head), and
+// where the grid is large. That saves their share of the SIMDs' time, 3% of the forward with one tile
+// and 1 to 6% with more and a large grid ([512, 8, 264, 64] 0.95 of the time). But workgroups that
+// end early draw later ones onto their CUs, and with few rounds of workgroups the uneven rest costs
+// more: D = 64, [12, 8, 904] 10% slower, [16, 8, 520] 11%, both near 1.5 rounds; past 8 rounds of the
+// three (D <= 32) or two workgroups of a CU, nothing of 46 shapes was slower: 24 workgroups for each of
+// 256 CUs. (From the grid, which the kernels have at hand: a flag of its own among the arguments took
+// 0.5 to 1% of the forward.)
+__device__ __forceinline__ bool idle_waves(uint32_t grid, uint32_t query_tiles) {
+    return query_tiles == 1u || grid >= 24u * 256u;
+}
+
 // A direct-to-LDS buffer load of BYTES (16 or 4) per lane: lane l's bytes at offset `off` of the
 // buffer land at dst + BYTES l, dst uniform across the wave; offsets past the buffer's range write
 // zeros. Counted by vmcnt like any load. (The 16-byte form is a gfx950 builtin that hipcc's host

@@ -227,6 +227,16 @@ def test_batch_sizes(hip, n):
     check(got, ref, "n=%d" % n)
 
 
+@pytest.mark.parametrize("n,h,sq,sk,d", [(2, 3, 33, 130, 32), (2, 3, 60, 65, 64), (3, 2, 139, 130, 32), (3, 2, 264, 70, 96),
+                                         (768, 4, 139, 30, 32), (520, 4, 300, 20, 64), (1600, 2, 200, 7, 16)])
+def test_waves_without_queries(hip, n, h, sq, sk, d):
+    """A last query tile that leaves one to three of a workgroup's four waves with no query: these
+    compute on zeros in small grids of several tiles a head, and only stage keys where a head has one
+    tile and in grids of 6144 workgroups (24 a CU) and more."""
+    got, ref = run(hip, n=n, h=h, sq=sq, sk=sk, d=d, seed=8, bk=64 if d == 64 else 32)
+    check(got, ref, "idle waves n=%d sq=%d sk=%d d=%d" % (n, sq, sk, d))
+
+
 @pytest.mark.parametrize("n,h,s,registers", [(512, 8, 96, 1), (128, 16, 128, 1), (96, 4, 200, 1),
                                               (64, 4, 300, 1), (256, 1, 416, 0), (256, 1, 448, 0)])
 def test_multi_pass_dkdv(hip, n, h, s, registers):
