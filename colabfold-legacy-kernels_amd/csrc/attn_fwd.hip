@@ -55,7 +55,7 @@ enum ItemOrder { kOrderRows = 0, kOrderHeads = 1, kOrderHeadPairs = 2 };
 //   boundary. The wave's two query blocks then take the rows of one parity each (block 0 the
 //   aligned ones), so that the 2-byte shift is known at compile time and costs no instruction;
 // - kBiasRegs: 2-byte loads of each lane's 16 keys, for what is left (a bias at an odd multiple of
-//   2 bytes with Sk even, or a head's bias of 2^31 bytes or more).
+//   2 bytes with Sk even, a head's bias of 2^31 bytes or more, or a short odd Sk: bias_mode).
 // Every Sk % 8 != 0 used to run kBiasRegs, whose 32 2-byte loads a tile and lane set the kernel's
 // time: the gated packed forward at [139, 139, 4, 4, 16] took 33.4 us and takes 16.3 (by columns), a
 // triangle attention block of 381 residues (4 heads of 32, with its two projections) 354 and 152.
@@ -813,11 +813,16 @@ __global__ __launch_bounds__(FwdTile<DP>::kThreads, DP == 32 ? 3 : 1) void attn_
 
 // BiasMode of a bias [H, Sq, Sk]. Direct-to-LDS loads take 32-bit offsets within a head's bias, and
 // the swizzled rows past Sq must not wrap: heads of 2^31 bytes or more go through registers.
-static int bias_mode(const void* bias, int64_t Sq, int64_t Sk) {
+// An odd Sk of one key tile that leaves more than kKillMax keys of it dead pays for them by rows
+// (kill_rows_lds): there 2-byte loads measured faster for Sk <= 16 (by 12 to 16% without a gate, 0 to
+// 18% with one) and, ungated at D <= 32, up to where the dead keys fall to kKillMax (10% at 23, 8% at
+// 39, 2 to 3% at 53 keys; gated they are 9 to 16% slower there). [4096, 4, 9, 64] gated 161 -> 132 us,
+// [4096, 4, 13, 32] ungated 77 -> 66.
+static int bias_mode(const void* bias, int64_t Sq, int64_t Sk, bool short_regs) {
     if (Sq * Sk * 2 >= ((int64_t)1 << 31) - 4) return kBiasRegs;
     const uintptr_t at = reinterpret_cast<uintptr_t>(bias);
     if (Sk % 2 == 0) return at % 4 == 0 ? kBiasDma : kBiasRegs;
-    return at % 2 == 0 ? kBiasDmaOdd : kBiasRegs;
+    return at % 2 == 0 && Sk > (short_regs ? 55 : 16) ? kBiasDmaOdd : kBiasRegs;
 }
 
 template <int DP, bool LSE, bool GATE, bool TRIM>
@@ -836,7 +841,7 @@ static int launch_fwd(hipStream_t stream, int device, const FwdArgs& a) {
     b.fqt = fast_div(qt);
     b.fn = fast_div(a.N);
     b.fh = fast_div(a.H);
-    const int bm = bias_mode(a.bias, a.Sq, a.Sk);
+    const int bm = bias_mode(a.bias, a.Sq, a.Sk, !GATE && DP == 32);
     stage_mark(stream, 0);
 #define CLK_FWD(BM_)                                                                               \
     if (bm == BM_) hipLaunchKernelGGL((attn_fwd_kernel<DP, LSE, GATE, TRIM, BM_>), dim3((unsigned)grid), \

@@ -2,7 +2,7 @@
 
 The forward reads its bias [H, Sq, Sk] in one of three ways, chosen by Sk and the address: rows on
 4-byte boundaries (Sk even) and rows of odd Sk, both through LDS, and 2-byte loads for the rest (Sk
-even at an odd element offset). The cases sit at the edges of a 64-key tile, where an odd row's
+even at an odd element offset; odd Sk up to 16, ungated at D <= 32 up to 55). The cases sit at the edges of a 64-key tile, where an odd row's
 last key lies past the tile, with no dead key, a few (among them key 63), and more than the
 tile-wide limit of 8 for single stores. With odd Sk the same values at an odd element offset, which
 swaps the roles of even and odd queries within the same kernel, must give the same bits.
@@ -32,7 +32,7 @@ def mask(kind, n, sk, rng):
 
 
 @pytest.mark.parametrize("kind", ["none", "few", "many"])
-@pytest.mark.parametrize("sq,sk,d", [(33, 1, 32), (5, 7, 8), (63, 63, 32), (64, 65, 16), (130, 127, 32), (129, 129, 32),
+@pytest.mark.parametrize("sq,sk,d", [(33, 1, 32), (5, 7, 8), (20, 15, 64), (20, 17, 64), (40, 55, 16), (40, 57, 16), (63, 63, 32), (64, 65, 16), (130, 127, 32), (129, 129, 32),
                                      (131, 191, 64), (37, 193, 96), (66, 130, 32), (65, 132, 32), (64, 134, 64),
                                      (257, 261, 32)])
 def test_bias_rows(hip, sq, sk, d, kind):
