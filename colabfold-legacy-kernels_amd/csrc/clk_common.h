@@ -104,16 +104,17 @@ __device__ __forceinline__ half8 lds_operand_tr(At at, int g, int lane16, int co
 }
 
 // Whether an attention kernel's waves that have no query (of a last tile that Sq cuts short) skip the
-// products and only stage keys: where every workgroup is such a one (a single query tile a head), and
-// where the grid is large. That saves their share of the SIMDs' time, 3% of the forward with one tile
-// and 1 to 6% with more and a large grid ([512, 8, 264, 64] 0.95 of the time). But workgroups that
+// products and only stage keys: where every workgroup is such a one, or every second (one or two query
+// tiles a head), and where the grid is large. That saves their share of the SIMDs' time, 3% of the
+// forward with one tile, 1 to 2% with two (Sq = 139 and 160) and 1 to 6% with more and a large grid
+// ([512, 8, 264, 64] 0.95 of the time). But workgroups that
 // end early draw later ones onto their CUs, and with few rounds of workgroups the uneven rest costs
 // more: D = 64, [12, 8, 904] 10% slower, [16, 8, 520] 11%, both near 1.5 rounds; past 8 rounds of the
 // three (D <= 32) or two workgroups of a CU, nothing of 46 shapes was slower: 24 workgroups for each of
 // 256 CUs. (From the grid, which the kernels have at hand: a flag of its own among the arguments took
 // 0.5 to 1% of the forward.)
 __device__ __forceinline__ bool idle_waves(uint32_t grid, uint32_t query_tiles) {
-    return query_tiles == 1u || grid >= 24u * 256u;
+    return query_tiles <= 2u || grid >= 24u * 256u;
 }
 
 // A direct-to-LDS buffer load of BYTES (16 or 4) per lane: lane l's bytes at offset `off` of the

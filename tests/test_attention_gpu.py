@@ -228,11 +228,13 @@ def test_batch_sizes(hip, n):
 
 
 @pytest.mark.parametrize("n,h,sq,sk,d", [(2, 3, 33, 130, 32), (2, 3, 60, 65, 64), (3, 2, 139, 130, 32), (3, 2, 264, 70, 96),
-                                         (768, 4, 139, 30, 32), (520, 4, 300, 20, 64), (1600, 2, 200, 7, 16)])
+                                         (260, 8, 264, 30, 32), (260, 8, 300, 20, 64), (260, 8, 330, 7, 16)])
 def test_waves_without_queries(hip, n, h, sq, sk, d):
     """A last query tile that leaves one to three of a workgroup's four waves with no query: these
     compute on zeros in small grids of several tiles a head, and only stage keys where a head has one
-    tile and in grids of 6144 workgroups (24 a CU) and more."""
+    or two and in grids of 6144 workgroups (24 a CU) and more. (dbias sums n rows, each with out's fp16
+    rounding in its delta, so its error grows with the root of n, and with 1 / sk: 5.5e-3 at 800 rows
+    of 7 keys, above the absolute bar; so the large grids here come from heads.)"""
     got, ref = run(hip, n=n, h=h, sq=sq, sk=sk, d=d, seed=8, bk=64 if d == 64 else 32)
     check(got, ref, "idle waves n=%d sq=%d sk=%d d=%d" % (n, sq, sk, d))
 
